@@ -330,3 +330,12 @@ def test_inertia_of_points_that_are_centroids(vh, oracle, metric):
         den = np.linalg.norm(x, axis=1) * np.linalg.norm(c, axis=1)
         want = np.sum(1.0 - dots / den)
         assert abs(got["inertia"] - want) <= 2e-7 * n + 2e-6 * abs(want)
+
+
+@pytest.mark.parametrize("k,dim", [(1, 1), (5, 31), (3, 32), (257, 33), (1000, 100), (2, 1023)])
+def test_read_returns_the_centroids_set(vh, k, dim):
+    """Centroids come back as they went in at widths with and without padding (contiguous rows)."""
+    c = np.arange(k * dim, dtype=np.float32).reshape(k, dim) - 7
+    st = vh.KMeansState(np.concatenate([c, c + 1]))
+    st.set_centroids(c)
+    np.testing.assert_array_equal(st.read()["centroids"], c)

@@ -743,6 +743,18 @@ __global__ __launch_bounds__(kKppSelectThreads) void k_kpp_select(const double *
     for (int d = t; d < dpad; d += kKppSelectThreads) dst[d] = src[d];
 }
 
+// Rows of dpad floats into contiguous rows of dim floats (dim < dpad), the layout of the caller's
+// centroid buffer.  The copy out is then one linear transfer: a strided one (hipMemcpy2D to pageable
+// memory) moves row by row, about 7 us a row: reading 1,024 x 96 centroids took 7.0 ms and takes
+// 0.1 ms, five Lloyd iterations at 500,000 x 96 with their read-out 12.7 -> 5.9 ms.
+__global__ __launch_bounds__(256) void k_rows_unpad(const float *__restrict__ in, size_t count, int dim, int dpad,
+                                                    float *__restrict__ out) {
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x) {
+        const size_t r = i / (size_t)dim;
+        out[i] = in[r * dpad + (i - r * dim)];
+    }
+}
+
 __global__ void k_fill(float *p, size_t count, float v) {
     const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
     if (i < count) p[i] = v;
@@ -765,7 +777,7 @@ struct vhip_kmeans {
     // they differ (the update, inertia and fix-up read them); craw: the centroids (the state),
     // cent: their assign rows (shifted, kpad rows with NaN padding)
     vh::DevBuf pts, praw, shift, pnorm, craw, cent, cnorm, cabs, cmax, assign, pos, inertia, counts, offsets, sorted,
-        shifts, partial, sums, exps, devmax, fix, nfix, best;
+        shifts, partial, sums, exps, devmax, fix, nfix, best, rows_out;
     const float *points() const { return shifted ? praw.as<float>() : pts.as<float>(); }
     vh::PinnedStager stager;
     vh::KernelTimer timer;
@@ -1011,21 +1023,6 @@ static int km_iterate(vhip_kmeans *K) {
     return VHIP_OK;
 }
 
-static int km_total_inertia(vhip_kmeans *K, float *out) {
-    const int nb = 256;
-    const size_t chunk = (K->n + nb - 1) / nb;
-    hipLaunchKernelGGL(k_sum_partial, dim3(nb), dim3(256), 0, K->stream, K->inertia.as<float>(), K->n, chunk,
-                       K->partial.as<double>());
-    VH_HIP(hipGetLastError());
-    std::vector<double> part(nb);
-    VH_HIP(hipMemcpyAsync(part.data(), K->partial.p, nb * sizeof(double), hipMemcpyDeviceToHost, K->stream));
-    VH_HIP(hipStreamSynchronize(K->stream));
-    double s = 0.0;
-    for (double v : part) s += v;
-    *out = (float)s;
-    return VHIP_OK;
-}
-
 // Seeded k-means++ (kmeans.rs:409-460): first centre uniform, then each next centre drawn
 // with probability proportional to the squared L2 distance to the nearest chosen centre.  The
 // draws (one 64-bit splitmix64 value per centre) are made on the host up front; every step then
@@ -1187,15 +1184,42 @@ int vhip_kmeans_read(vhip_kmeans *K, float *centroids, int32_t *assign, int64_t 
     std::lock_guard<std::mutex> lock(K->mu);
     VH_CHECK(open_device(K->dev));
     hipStream_t s = K->stream;
-    if (centroids && K->k)
-        VH_HIP(hipMemcpy2DAsync(centroids, K->dim * sizeof(float), K->craw.p, K->dpad * sizeof(float),
-                                K->dim * sizeof(float), K->k, hipMemcpyDeviceToHost, s));
-    if (assign && K->assigned)
-        VH_HIP(hipMemcpyAsync(assign, K->assign.p, K->n * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    std::vector<int32_t> c32(K->k);
-    std::vector<float> sh(K->k);
-    if (K->assigned && K->k) {
+    // the inertia's sum first, so that one wait covers it and the copies
+    constexpr int kInertiaParts = 256;
+    std::vector<double> part;
+    if (inertia && K->assigned) {
+        part.resize(kInertiaParts);
+        const size_t chunk = (K->n + kInertiaParts - 1) / kInertiaParts;
+        hipLaunchKernelGGL(k_sum_partial, dim3(kInertiaParts), dim3(256), 0, s, K->inertia.as<float>(), K->n, chunk,
+                           K->partial.as<double>());
+        VH_HIP(hipGetLastError());
+        VH_HIP(hipMemcpyAsync(part.data(), K->partial.p, kInertiaParts * sizeof(double), hipMemcpyDeviceToHost, s));
+    }
+    const size_t cbytes = K->k * K->dim * sizeof(float);
+    const void *crows = K->craw.p;
+    if (centroids && K->k && K->dim != K->dpad) {
+        VH_CHECK(K->rows_out.ensure(K->dev, cbytes));
+        const size_t blocks = std::min<size_t>(4096, (K->k * K->dim + 255) / 256);
+        hipLaunchKernelGGL(k_rows_unpad, dim3((unsigned)blocks), dim3(256), 0, s, K->craw.as<float>(), K->k * K->dim,
+                           (int)K->dim, (int)K->dpad, K->rows_out.as<float>());
+        VH_HIP(hipGetLastError());
+        crows = K->rows_out.p;
+    }
+    const bool want_assign = assign && K->assigned;
+    if (centroids && K->k && want_assign)
+        VH_CHECK(K->stager.d2h_pair(centroids, crows, cbytes, assign, K->assign.p, K->n * sizeof(int32_t), s));
+    else if (centroids && K->k)
+        VH_CHECK(K->stager.d2h(centroids, crows, cbytes, s));
+    else if (want_assign)
+        VH_CHECK(K->stager.d2h(assign, K->assign.p, K->n * sizeof(int32_t), s));
+    std::vector<int32_t> c32;
+    std::vector<float> sh;
+    if (K->assigned && K->k && counts) {
+        c32.resize(K->k);
         VH_HIP(hipMemcpyAsync(c32.data(), K->counts.p, K->k * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    }
+    if (K->assigned && K->k && (shifts || max_shift)) {
+        sh.resize(K->k);
         VH_HIP(hipMemcpyAsync(sh.data(), K->shifts.p, K->k * sizeof(float), hipMemcpyDeviceToHost, s));
     }
     VH_HIP(hipStreamSynchronize(s));
@@ -1210,8 +1234,9 @@ int vhip_kmeans_read(vhip_kmeans *K, float *centroids, int32_t *assign, int64_t 
         *max_shift = m;
     }
     if (inertia) {
-        *inertia = 0.0f;
-        if (K->assigned) VH_CHECK(km_total_inertia(K, inertia));
+        double sum = 0.0;
+        for (double v : part) sum += v;
+        *inertia = (float)sum;
     }
     return VHIP_OK;
 }
