@@ -1,0 +1,81 @@
+"""Small query batches under the vector-ALU metrics and packed Hamming (knn_rows.hip).
+
+A score's terms are summed in the batch kernels' order, so a query gets the same ids and the same
+distances, bit for bit, whether it is searched in a small batch or within a large one; the large
+batches are held to the oracle elsewhere.  Sizes sit at the edges of the kernels: query tiles of 4 and
+16, the 64-query limit, 32-dimension chunks and the two chunk widths of the batch kernel, workgroups
+of 256 rows, the 8,192-row first round and one more round."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def vh():
+    import vector_hip
+
+    assert vector_hip.CudaDeviceContext.device_count() >= 1
+    return vector_hip
+
+
+@pytest.mark.parametrize("metric", ["Manhattan", "Minkowski", "Chebyshev", "Hamming", "Mahalanobis", "Jaccard",
+                                    "Hellinger"])
+@pytest.mark.parametrize("n,dim,k", [(3, 5, 10), (257, 32, 1), (8193, 33, 7), (20_001, 65, 100), (16_385, 128, 10),
+                                     (140_000, 129, 10), (9000, 200, 300)])
+def test_small_batches_equal_large_ones(vh, metric, n, dim, k):
+    rng = np.random.default_rng(n + dim)
+    base = rng.uniform(-1, 1, (n, dim)).astype(np.float32)
+    base[rng.integers(0, n, n // 3)] = base[rng.integers(0, n, n // 3)]  # equal rows: ties by id
+    if metric == "Hamming":
+        base = np.round(base * 2)
+    q = np.concatenate([base[:2], rng.uniform(-1, 1, (78, dim)).astype(np.float32)])
+    eng = vh.CudaKnnEngine(base, dim, vh.DistanceMetric[metric])
+    ids, dist, lens = eng.search_batch_arrays(q, k)
+    kk = min(k, n)
+    for nq in (1, 4, 5, 16, 17, 64):
+        i2, d2, l2 = eng.search_batch_arrays(q[:nq], k)
+        np.testing.assert_array_equal(i2[:, :kk], ids[:nq, :kk])
+        np.testing.assert_array_equal(d2[:, :kk], dist[:nq, :kk])
+        np.testing.assert_array_equal(l2, lens[:nq])
+
+
+@pytest.mark.parametrize("metric", ["Manhattan", "Minkowski"])
+def test_rows_and_queries_with_nan(vh, metric):
+    """A row with a NaN never appears, a query with one finds nothing, in small and large batches alike."""
+    rng = np.random.default_rng(3)
+    base = rng.uniform(-1, 1, (9000, 40)).astype(np.float32)
+    bad = rng.random(9000) < 0.999
+    base[bad, 7] = np.nan  # fewer finite rows than k
+    q = rng.uniform(-1, 1, (80, 40)).astype(np.float32)
+    q[1, 0] = np.nan
+    eng = vh.CudaKnnEngine(base, 40, vh.DistanceMetric[metric])
+    ids, dist, _ = eng.search_batch_arrays(q, 30)
+    good = np.flatnonzero(~bad)
+    assert 0 < good.size < 30
+    for r in (0, 2, 79):
+        assert sorted(ids[r, :good.size]) == good.tolist()
+        assert np.all(ids[r, good.size:] == 0xFFFFFFFF) and np.all(np.isnan(dist[r, good.size:]))
+    assert np.all(ids[1] == 0xFFFFFFFF)
+    for nq in (2, 16, 33):
+        i2, d2, _ = eng.search_batch_arrays(q[:nq], 30)
+        np.testing.assert_array_equal(i2, ids[:nq])
+        np.testing.assert_array_equal(d2, dist[:nq])
+
+
+@pytest.mark.parametrize("words", [1, 2, 3, 8, 9, 32])
+@pytest.mark.parametrize("n,k", [(5, 10), (257, 3), (20_000, 100), (300_001, 10)])
+def test_hamming_small_batches(vh, words, n, k):
+    rng = np.random.default_rng(words * 1000 + n)
+    codes = rng.integers(0, 1 << 32, (n, words), dtype=np.uint64).astype(np.uint32)
+    codes[rng.integers(0, n, n // 3)] = codes[0]  # massive ties
+    q = np.concatenate([codes[:2], rng.integers(0, 1 << 32, (68, words), dtype=np.uint64).astype(np.uint32)])
+    eng = vh.HammingKnnEngine(codes)
+    ids, dist, _ = eng.search_batch_arrays(q, k)
+    kk = min(k, n)
+    d0 = np.array([np.sum([bin(int(w)).count("1") for w in q[0] ^ codes[i]]) for i in ids[0, :kk]])
+    np.testing.assert_array_equal(dist[0, :kk], d0)
+    for nq in (1, 4, 5, 17, 64):
+        i2, d2, _ = eng.search_batch_arrays(q[:nq], k)
+        np.testing.assert_array_equal(i2[:, :kk], ids[:nq, :kk])
+        np.testing.assert_array_equal(d2[:, :kk], dist[:nq, :kk])

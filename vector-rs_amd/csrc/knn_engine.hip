@@ -84,6 +84,7 @@ struct vhip_knn {
     vh::DevBuf base8;  // packed Hamming on the fp4 matrix cores: one +1/-1 nibble per code bit
     bool ham8 = false;
     bool ham_wide = false;  // filter rounds may use the 1024-column fp4 kernel (codes <= 256 bits)
+    bool ham_small = false;  // small batches may scan the packed codes (no kernel was asked for by name)
     std::mutex mu;
     vh::Workspace ws;
     vh::PinnedStager stager;
@@ -132,17 +133,22 @@ constexpr int kRoundGrowth = 4;
 // k = 100 three rounds.)  A larger first round costs more in its merge (32,768 rows: 27 us against
 // about 12) than the fewer passes save.
 constexpr size_t kSmallDenseRows = 8192;
+// Batches the row-per-lane scan serves above that size start with this many dense rows at least: the
+// scan's small rounds cost about as much as its launches and merges, whatever their rows (L1 500k x 128,
+// 700 queries 1906 -> 1862 us, 4,096 queries 10528 -> 10163; L-inf 150,001 x 100, 700 queries 625 -> 610).
+constexpr size_t kRowScanFirst = 2048;
 
-static std::vector<Round> plan_rounds(size_t n, size_t k, bool gemm, int dpad, int growth, bool small = false) {
+static std::vector<Round> plan_rounds(size_t n, size_t k, bool dense0, int dpad, int growth, bool small = false,
+                                      size_t first = 256) {
     std::vector<Round> r;
     if (n == 0) return r;
     const size_t kk = std::max<size_t>(k, 1);
-    size_t b0 = std::min(n, round_up(std::max<size_t>(256, 20 * kk), kRowAlign));
+    size_t b0 = std::min(n, round_up(std::max<size_t>(first, 20 * kk), kRowAlign));
     // A base within the candidate capacity's floor (round_cap) is scored in one dense round: its
     // later rounds would cost more launches than rows (the IVF coarse probe: 1,024 centroids).
     if (n <= std::max<size_t>(2048, 32 * kk)) b0 = n;
     if (small) b0 = n <= 2 * kSmallDenseRows ? n : std::max(b0, kSmallDenseRows);
-    r.push_back({0, (long)b0, gemm, (long)kRowAlign, (long)kRowAlign});
+    r.push_back({0, (long)b0, dense0, (long)kRowAlign, (long)kRowAlign});
     const int slots = gemm_slots(dpad);
     const size_t cap_floor = std::max<size_t>({2048, 32 * kk, b0});
     size_t seen = b0;
@@ -180,9 +186,9 @@ static long balanced_item(long cap_item, long rows, int n_ctiles, int wgs, long 
 // the ~3 k expected passes of a filter round.  A query that still overflows is re-run with a
 // capacity equal to the largest round.
 
-static int round_cap(size_t n, size_t k, bool gemm, int dpad, bool small) {
+static int round_cap(size_t n, size_t k, int dpad, bool small) {
     size_t cap = std::max<size_t>(2048, 32 * std::max<size_t>(k, 1));
-    for (const Round &r : plan_rounds(n, k, gemm, dpad, kRoundGrowth, small))
+    for (const Round &r : plan_rounds(n, k, true, dpad, kRoundGrowth, small))
         if (r.rb == 0) cap = std::max(cap, (size_t)(r.re - r.rb));
     return (int)round_up(cap, kRowAlign);
 }
@@ -323,10 +329,8 @@ static RunBufs carve_run(Arena &A, const vhip_knn *E, size_t nq, int kc, int cap
     B.mflag = A.take<uint32_t>(nq);
     B.nflag = A.take<uint32_t>(2);
     if (E->ham8) B.q8 = A.take<int8_t>(round_up(nq, kTileCols) * ham_mfma_row_bytes((int)E->dpad));
-    if (is_gemm_metric(E->metric)) {
-        // any run of at most kSmallPadQueries of these queries may take the small-batch scan
-        B.spad = A.take<uint32_t>(std::min<size_t>(nq, kSmallPadQueries) * kSmallPadStride);
-    }
+    // any run of at most kSmallPadQueries of these queries may take the small-batch scan
+    B.spad = A.take<uint32_t>(std::min<size_t>(nq, kSmallPadQueries) * kSmallPadStride);
     return B;
 }
 
@@ -347,21 +351,28 @@ static std::vector<Round> split_rounds(const std::vector<Round> &r, long max_row
     return out;
 }
 
-// The round plan of a search over nq queries: the small-batch plan for at most kSmallCols queries
-// on the GEMM metrics (not the direct-form re-runs).
-static bool small_plan(const vhip_knn *E, size_t nq, bool direct) {
-    return is_gemm_metric(E->metric) && !direct && !E->ham8 &&
-           small_batch((int)std::min<size_t>(nq, 1 << 20), (int)E->dpad, E->n);
+// Whether a run over nq queries takes the small-batch scans, which count FILTER candidates on spread
+// counters (not the direct-form re-runs): the MFMA one for the GEMM metrics (small_batch), the
+// row-per-lane one for the others.
+static bool small_scan_run(const vhip_knn *E, size_t nq, bool direct) {
+    if (direct) return false;
+    if (is_gemm_metric(E->metric)) return small_batch((int)std::min<size_t>(nq, 1 << 20), (int)E->dpad, E->n);
+    if (E->metric == HAMMING_PACKED) return E->ham_small && nq <= (size_t)kHamSmallQueries;
+    return nq <= (size_t)kValuSmallQueries;
 }
+// ... which run on the small-batch round plan.
+static bool small_plan(const vhip_knn *E, size_t nq, bool direct) { return small_scan_run(E, nq, direct); }
 
 // The candidate count a run starts from: the first round's rows when that round is dense (every
 // score is written), else 0.
-static uint32_t first_count(const std::vector<Round> &rounds, const vhip_knn *E) {
-    const bool dense0 = !rounds.empty() && (rounds[0].dense || (E->ham8 && rounds[0].rb == 0));
-    return dense0 ? (uint32_t)(rounds[0].re - rounds[0].rb) : 0u;
+static uint32_t first_count(const std::vector<Round> &rounds) {
+    return !rounds.empty() && rounds[0].dense ? (uint32_t)(rounds[0].re - rounds[0].rb) : 0u;
 }
-static std::vector<Round> run_plan(const vhip_knn *E, int k, bool gemm, bool small, long max_round_rows) {
-    return split_rounds(plan_rounds(E->n, (size_t)k, gemm, (int)E->dpad, kRoundGrowth, small), max_round_rows);
+// The rounds of a run.  The first is dense on every path but the popcount batch kernel's.
+static std::vector<Round> run_plan(const vhip_knn *E, int k, bool small, long max_round_rows) {
+    const bool dense0 = E->metric != HAMMING_PACKED || E->ham8 || small;
+    const size_t first = is_gemm_metric(E->metric) || E->metric == HAMMING_PACKED ? 256 : kRowScanFirst;
+    return split_rounds(plan_rounds(E->n, (size_t)k, dense0, (int)E->dpad, kRoundGrowth, small, first), max_round_rows);
 }
 
 // Runs all rounds for nq prepared queries; results stay in B.topk (row stride kc) / B.have.
@@ -374,10 +385,12 @@ static int run_rounds(vhip_knn *E, const QueryRows &Q, int nq, int k, int kc, in
                       const RunBufs &B, long max_round_rows, bool timed, bool reset_done = false) {
     hipStream_t s = E->stream;
     const bool gemm = is_gemm_metric(E->metric) && !direct;
-    const std::vector<Round> rounds = run_plan(E, k, gemm, small, max_round_rows);
+    const std::vector<Round> rounds = run_plan(E, k, small, max_round_rows);
     if (!reset_done)
-        launch_topk_init(nq, B.tau, B.have, B.cnt, B.flags, B.mflag, B.nflag, first_count(rounds, E), B.spad, s);
-    if (E->ham8) {
+        launch_topk_init(nq, B.tau, B.have, B.cnt, B.flags, B.mflag, B.nflag, first_count(rounds), B.spad, s);
+    const bool small_scan = small_scan_run(E, (size_t)nq, direct);
+    const bool ham8 = E->ham8 && !small_scan;
+    if (ham8) {
         // the queries' +1/-1 nibbles, rows padded to the 128-query tiles
         const size_t rows = round_up((size_t)nq, kTileCols);
         launch_ham_expand((const uint32_t *)Q.qpad, (size_t)nq, (int)E->dpad, (int)E->dpad, rows, false, B.q8, s);
@@ -385,21 +398,20 @@ static int run_rounds(vhip_knn *E, const QueryRows &Q, int nq, int k, int kc, in
     for (size_t ri = 0; ri < rounds.size(); ++ri) {
         const Round &rd = rounds[ri];
         const long rb = rd.rb, re = rd.re;
-        const bool dense = rd.dense || (E->ham8 && rb == 0);
+        const bool dense = rd.dense;
         // Algorithmic work per launch: 2*Q*rows*D flops (GEMM metrics), Q*rows*D element
         // operations (VALU metrics) or Q*rows*words word operations (packed Hamming); bytes
         // are the base rows and queries each launch must read once.  The direct-form passes
         // are not timed (they are not the engine's scan).
         const double rows = (double)(re - rb);
         const double work = gemm ? 2.0 * nq * rows * (double)E->dim
-                                 : (E->ham8 ? 2.0 * nq * rows * 2.0 * (double)ham_mfma_row_bytes((int)E->dpad)
+                                 : (ham8 ? 2.0 * nq * rows * 2.0 * (double)ham_mfma_row_bytes((int)E->dpad)
                                             : (double)nq * rows * (double)E->dim);
-        const double bytes = E->ham8 ? (rows + nq) * (double)ham_mfma_row_bytes((int)E->dpad)  // expanded codes
+        const double bytes = ham8 ? (rows + nq) * (double)ham_mfma_row_bytes((int)E->dpad)  // expanded codes
                                      : rows * E->dim * 4.0 + (double)nq * E->dim * 4.0;
         if (dense && ri > 0) launch_fill_u32(B.cnt, (size_t)nq, (uint32_t)(re - rb), s);
-        // the small-batch scan's FILTER rounds count candidates on B.spad (kSmallPadStride apart)
-        const bool small_scan = !E->ham8 && gemm && small_batch(nq, (int)E->dpad, E->n);
-        const bool spread = small_scan && !rd.dense;
+        // the small-batch scans' FILTER rounds count candidates on B.spad (kSmallPadStride apart)
+        const bool spread = small_scan && !dense;
         const int t = (direct || !timed) ? -1 : E->timer.begin(s);
         // the narrow resident-tile kernel (gemm_narrow) works in 512-row stages on 32-column tiles
         const bool narrow = gemm && gemm_narrow((int)E->dpad);
@@ -407,7 +419,7 @@ static int run_rounds(vhip_knn *E, const QueryRows &Q, int nq, int k, int kc, in
                               ? balanced_item(rd.item_rows, re - rb, ceil_div(nq, gemm_filter_cols((int)E->dpad)),
                                               E->grid_cap / 2, narrow ? 512 : kRowAlign)
                               : (narrow ? std::max<long>(rd.item_rows, 512) : rd.item_rows);
-        if (E->ham8) {
+        if (ham8) {
             // fp4 matrix-core Hamming: 2 K operations per (query, row), K = the padded code bits.
             // Items up to 32768 rows where the slot rule allows: each spreads its query-tile fill
             // and flush over more 512-row stages (5% faster at 10M x 256 bits than 8192)
@@ -428,7 +440,7 @@ static int run_rounds(vhip_knn *E, const QueryRows &Q, int nq, int k, int kc, in
                 launch_ham_mfma(dense, hitem, E->base8.as<int8_t>(), B.q8, (int)E->dpad, B.tau, nq, rb, re, B.cand,
                                 B.cnt, cap, E->grid_cap, s);
             }
-        } else if (small_scan)
+        } else if (gemm && small_scan)
             launch_small_scan(E->metric, rd.dense, E->base.as<float>(), E->norm.as<float>(), Q.qpad, Q.qnorm, B.tau,
                               nq, (int)E->dpad, rb, re, rd.plan_rows ? rd.plan_rows : re - rb, B.cand, B.spad, cap,
                               E->grid_cap, s);
@@ -436,15 +448,15 @@ static int run_rounds(vhip_knn *E, const QueryRows &Q, int nq, int k, int kc, in
             launch_gemm_filter(E->metric, rd.dense, item, E->base.as<float>(), E->norm.as<float>(), Q.qpad, Q.qnorm,
                                B.tau, nq, (int)E->dpad, rb, re, B.cand, B.cnt, cap, E->norm_max, E->norm_min,
                                E->grid_cap, s);
-        else if (E->metric == HAMMING_PACKED)
+        else if (E->metric == HAMMING_PACKED && !small_scan)
             launch_hamming_filter(E->base.as<uint32_t>(), (const uint32_t *)Q.qpad, B.tau, nq, (int)E->dpad, rb, re,
                                   B.cand, B.cnt, cap, E->grid_cap, s);
         else if (direct)
-            launch_valu_filter(L2, direct_rows(E), direct_shift(E), Q.qraw, B.tau, nq, (int)E->dim, (int)E->dpad, rb,
-                               re, B.cand, B.cnt, cap, E->grid_cap, s);
+            launch_row_scan(L2, dense, direct_rows(E), direct_shift(E), Q.qraw, B.tau, nq, (int)E->dim, (int)E->dpad,
+                            rb, re, B.cand, B.cnt, 1, cap, s);
         else
-            launch_valu_filter(E->metric, E->base.as<float>(), nullptr, Q.qpad, B.tau, nq, (int)E->dim, (int)E->dpad,
-                               rb, re, B.cand, B.cnt, cap, E->grid_cap, s);
+            launch_row_scan(E->metric, dense, E->base.p, nullptr, Q.qpad, B.tau, nq, (int)E->dim, (int)E->dpad, rb,
+                            re, B.cand, spread ? B.spad : B.cnt, spread ? kSmallPadStride : 1, cap, s);
         if (t >= 0) E->timer.end(t, s, work, bytes);
         VH_HIP(hipGetLastError());
         // the last round counts the standing margin flags into nflag[1]
@@ -452,18 +464,19 @@ static int run_rounds(vhip_knn *E, const QueryRows &Q, int nq, int k, int kc, in
         launch_topk_merge(nq, k, kc, B.cand, spread ? B.spad : B.cnt, spread ? kSmallPadStride : 1, cap,
                           E->perm.as<uint32_t>(), B.topk, B.have, B.tau, B.flags,
                           B.nflag, gemm ? Q.qerr : nullptr, B.mflag, last && gemm ? B.nflag + 1 : nullptr,
-                          dense && re - rb > 4096, s);
+                          !gemm, dense && re - rb > 4096, s);
         VH_HIP(hipGetLastError());
     }
     return VHIP_OK;
 }
 
-// Capacity of a candidate list that no round can overflow: the largest round's rows, of either
-// round plan.
-static int full_cap(const vhip_knn *E, size_t k, bool gemm) {
+// Capacity of a candidate list that no round can overflow: the largest round's rows, of any round
+// plan.
+static int full_cap(const vhip_knn *E, size_t k) {
     long big = k;
-    for (int sm = 0; sm < 2; ++sm)
-        for (const Round &rd : plan_rounds(E->n, k, gemm, (int)E->dpad, kRoundGrowth, sm == 1))
+    for (int sm = 0; sm < 3; ++sm)
+        for (const Round &rd : plan_rounds(E->n, k, true, (int)E->dpad, kRoundGrowth, sm == 1,
+                                           sm == 2 ? kRowScanFirst : 256))
             big = std::max(big, rd.re - rd.rb);
     return (int)round_up((size_t)big, kRowAlign);
 }
@@ -499,9 +512,8 @@ static RerunMem carve_rerun(Arena &A, const vhip_knn *E, size_t nidx, size_t per
 static int rerun_queries(vhip_knn *E, const QueryRows &Q, const std::vector<uint32_t> &idx, int k, int kc,
                          bool direct, const RunBufs &M, const Arena *fixed, uint2 *cand, size_t cand_slots) {
     hipStream_t s = E->stream;
-    const bool gemm = is_gemm_metric(E->metric) && !direct;
     const int kc_run = direct ? k : kc;
-    const int cap_big = full_cap(E, (size_t)k, gemm);
+    const int cap_big = full_cap(E, (size_t)k);
     const int dp = (int)E->dpad;
     size_t per_batch = idx.size();
     int cap = cap_big;
@@ -738,6 +750,7 @@ static int engine_create(const void *base, size_t n, size_t dim, int metric, int
             const char *env = std::getenv("VHIP_HAMMING_KERNEL");
             E->ham_wide = ham_wide_supported((int)E->dpad) && !(env && std::strcmp(env, "fp4-tile") == 0);
         }
+        E->ham_small = metric == HAMMING_PACKED && !std::getenv("VHIP_HAMMING_KERNEL");
         uint32_t nonint = 1;
         VH_HIP(hipMemcpyAsync(&nonint, flag.p, sizeof(uint32_t), hipMemcpyDeviceToHost, E->stream));
         if (norm_kind_of(metric)) {
@@ -813,10 +826,10 @@ static int engine_search_locked(vhip_knn *E, const void *d_queries, size_t nq, s
     size_t batch = std::min(nq, kQueryBatch);
     // every batch of the call takes the plan its first does: the buffers are sized for that plan
     bool small = small_plan(E, batch, false);
-    int cap = round_cap(E->n, ek, gemm, (int)E->dpad, small);
+    int cap = round_cap(E->n, ek, (int)E->dpad, small);
     if (scratch && small && batch_bytes(E, batch, kc, cap, true) > scratch_bytes) {
         small = false;
-        cap = round_cap(E->n, ek, gemm, (int)E->dpad, false);
+        cap = round_cap(E->n, ek, (int)E->dpad, false);
     }
     if (scratch) {
         // the largest batch whose buffers and re-run reserve fit the scratch region
@@ -873,7 +886,7 @@ static int engine_search_locked(vhip_knn *E, const void *d_queries, size_t nq, s
         }
         // the batch's run starts here too (search_prepared's first run_rounds skips its reset)
         rp.init = {bm.B.tau, bm.B.have, bm.B.cnt, bm.B.flags, bm.B.mflag, bm.B.nflag, bm.B.spad,
-                   first_count(run_plan(E, kk, gemm, small, 0), E)};
+                   first_count(run_plan(E, kk, small, 0))};
         launch_rows_prep(rp, E->stream);
         VH_HIP(hipGetLastError());
         const QueryRows Q{bm.qpad, bm.qnorm, bm.qerr, E->shifted ? bm.qraw : bm.qpad};

@@ -1,235 +1,17 @@
-// knn_valu.hip -- non-contraction metrics on the vector ALUs, fused with the threshold
-// filter of the round/merge top-k (topk.hip).
-//
-// Replaces the metric switch of knn_compute_distance_matrix (vector-cuda/src/kernels/knn.cu:84-141,
-// 175-195) for squared L2 in direct form (the fallback of the GEMM-form L2 search), L1,
-// Minkowski p=3, L-inf, thresholded Hamming, Mahalanobis (sqrt of direct L2), weighted Jaccard
-// and Hellinger (direct L2 of sqrt|x|, then sqrt(0.5 * sum)).  Each lane owns
-// one query held in registers; a workgroup of 256 lanes streams tiles of base rows through LDS and
-// every wave reads each base element as a broadcast ds_read_b128 (all lanes the same address), so a
-// base element costs two VALU operations per query (sub + add/max with the |x| modifier).  Values
-// are computed in the direct form of the reference CPU engine (scalar.rs:81-263), so reported
-// distances follow it closely.
+// knn_valu.hip -- k-means assignment on the vector ALUs: the metrics that are no matrix product
+// (kmeans.cu:172-271), the direct-form fix-up of the certified MFMA assignment, and small point sets.
+// Each lane owns a point (or a slice of one) in registers and centroid tiles are broadcast from LDS or
+// streamed through L1.  Values are in the direct form of the reference CPU engine (scalar.rs:81-263).
 #include <algorithm>
 
+#include "valu_metrics.h"
 #include "vh_common.h"
 
 namespace vh {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-constexpr int kValuRows = 16;             // base rows per LDS tile
-constexpr long kValuItemRowsMax = 2048;   // base rows per work item (large rounds)
-
-// k-means Hellinger: centroids are means of the raw data, so sqrt(|x|) of the centroid
-// side is taken in the loop (the point side holds sqrt(|p|)).
-constexpr int HELL_RAW = 11;
-
-template <int M>
-__device__ __forceinline__ void accum(float &a, float &b, float q, float x) {
-    if constexpr (M == HELL_RAW) {
-        const float d = q - sqrtf(fabsf(x));
-        a = fmaf(d, d, a);
-    } else if constexpr (M == L1) {
-        a += fabsf(q - x);
-    } else if constexpr (M == L2 || M == MAHA || M == HELL) {
-        const float d = q - x;
-        a = fmaf(d, d, a);
-    } else if constexpr (M == LINF) {
-        a = fmaxf(a, fabsf(q - x));
-    } else if constexpr (M == MINK) {
-        const float d = fabsf(q - x);
-        a = fmaf(d * d, d, a);
-    } else if constexpr (M == HAMF) {
-        a += fabsf(q - x) > 1e-6f ? 1.0f : 0.0f;
-    } else if constexpr (M == DOT) {
-        a = fmaf(q, x, a);
-    } else if constexpr (M == COS) {  // dot product and the row's squared norm
-        a = fmaf(q, x, a);
-        b = fmaf(x, x, b);
-    } else {  // JACC: q holds |q|
-        const float ax = fabsf(x);
-        a += fminf(q, ax);
-        b += fmaxf(q, ax);
-    }
-}
-
-// Two consecutive elements; L-inf takes both in one max of three (|.| source modifiers).
-template <int M>
-__device__ __forceinline__ void accum2(float &a, float &b, float q0, float q1, float x0, float x1) {
-    if constexpr (M == LINF) {
-        a = fmaxf(a, fmaxf(fabsf(q0 - x0), fabsf(q1 - x1)));
-    } else {
-        accum<M>(a, b, q0, x0);
-        accum<M>(a, b, q1, x1);
-    }
-}
-
-template <int M>
-__device__ __forceinline__ float finish(float a, float b) {
-    if constexpr (M == MINK) return cbrtf(a);
-    else if constexpr (M == MAHA) return sqrtf(a);
-    else if constexpr (M == HELL || M == HELL_RAW) return sqrtf(0.5f * a);
-    else if constexpr (M == JACC) return b <= 1e-9f ? 0.0f : 1.0f - a / b;
-    else return a;
-}
-
-// DC: dimensions per chunk held in registers (64 or 128).  A wave serves 64 queries: lane (p, h)
-// holds queries 2p and 2p + 1 of its wave's group over half h of each chunk (DC / 2 dimensions of
-// each), so every broadcast tile read feeds two queries and a row costs DC / 8 LDS reads per lane,
-// half of what one query per lane over the whole chunk needs.  After a tile the two halves meet
-// with one cross-half exchange per row, and lane (p, h) finishes and filters query 2p + h.
-template <int M, int DC>
-__global__ __launch_bounds__(256) void k_valu_filter(const float *__restrict__ base, const float *__restrict__ shift,
-                                                     const float *__restrict__ qry, const float *__restrict__ tau,
-                                                     int nq, int dpad, long row_begin, long row_end, int n_qtiles,
-                                                     int n_items, long item_rows, uint2 *__restrict__ cand,
-                                                     uint32_t *__restrict__ cnt, int cap) {
-    constexpr int V4 = DC / 4, HD = DC / 2, H4 = HD / 4;
-    // rows interleaved per tile read: 4, or 2 for L-inf, whose max3 chains gain nothing from more
-    // (L1 at 500k x 128, Q = 4096: 10.90 ms at 4 rows, 11.09 at 2; L-inf 10.82 at 2, 10.90 at 4)
-    constexpr int RI = M == LINF ? 2 : 4;
-    __shared__ floatx4 tile[kValuRows * V4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int h = lane >> 5, pq = lane & 31;
-    const int nchunks = (dpad + DC - 1) / DC;
-    const int G = gridDim.x, g8 = G >> 3;
-    const int slot = (blockIdx.x & 7) * g8 + (blockIdx.x >> 3);
-
-    for (int item = slot; item < n_items; item += G) {
-        const int qtile = item % n_qtiles;
-        const long chunk = item / n_qtiles;
-        const int q0 = qtile * 256 + wave * 64 + 2 * pq;  // this lane's query pair
-        const int q = q0 + h;                              // the query it finishes
-        const bool qv = q < nq;
-        const float tq = qv ? tau[q] : -INFINITY;
-        const long r_lo = row_begin + chunk * item_rows;
-        const long r_hi = min(r_lo + item_rows, row_end);
-
-        float qr[2][HD];
-        auto load_q = [&](int c) {
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const bool v = q0 + e < nq;
-#pragma unroll
-                for (int i = 0; i < H4; ++i) {
-                    const int d = c * DC + h * HD + 4 * i;
-                    floatx4 x = (v && d < dpad) ? *(const floatx4 *)(qry + (long)(q0 + e) * dpad + d)
-                                                : floatx4{0, 0, 0, 0};
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) qr[e][4 * i + j] = (M == JACC) ? fabsf(x[j]) : x[j];
-                }
-            }
-        };
-        if (nchunks == 1) load_q(0);
-
-        for (long rs = r_lo; rs < r_hi; rs += kValuRows) {
-            float a[2][kValuRows], b[2][kValuRows];
-#pragma unroll
-            for (int r = 0; r < kValuRows; ++r) a[0][r] = a[1][r] = b[0][r] = b[1][r] = 0.0f;
-            for (int c = 0; c < nchunks; ++c) {
-                if (nchunks > 1) load_q(c);
-                __syncthreads();
-                for (int i = tid; i < kValuRows * V4; i += 256) {
-                    const int row = i / V4, c4 = i % V4;
-                    const long r = rs + row;
-                    const int d = c * DC + 4 * c4;
-                    floatx4 v = (r < r_hi && d < dpad) ? *(const floatx4 *)(base + r * (long)dpad + d)
-                                                       : floatx4{0, 0, 0, 0};
-                    if (shift && d < dpad) v += *(const floatx4 *)(shift + d);
-                    tile[i] = v;
-                }
-                __syncthreads();
-                // RI rows at a time: 2 RI independent accumulation chains per element
-#pragma unroll
-                for (int r = 0; r < kValuRows; r += RI) {
-#pragma unroll
-                    for (int i = 0; i < H4; ++i) {
-                        floatx4 x[RI];
-#pragma unroll
-                        for (int u = 0; u < RI; ++u) x[u] = tile[(r + u) * V4 + h * H4 + i];
-#pragma unroll
-                        for (int j = 0; j < 4; j += 2)
-#pragma unroll
-                            for (int u = 0; u < RI; ++u)
-#pragma unroll
-                                for (int e = 0; e < 2; ++e)
-                                    accum2<M>(a[e][r + u], b[e][r + u], qr[e][4 * i + j], qr[e][4 * i + j + 1],
-                                              x[u][j], x[u][j + 1]);
-                    }
-                }
-            }
-            const int nvalid = (int)min((long)kValuRows, r_hi - rs);
-#pragma unroll
-            for (int r = 0; r < kValuRows; ++r) {
-                // the partner half needs the other query's partial sums; this lane keeps its own
-                const float sa = __shfl_xor(h ? a[0][r] : a[1][r], 32, 64);
-                const float oa = h ? a[1][r] : a[0][r];
-                float sb = 0.0f, ob = 0.0f;
-                if constexpr (M == JACC || M == COS) {
-                    sb = __shfl_xor(h ? b[0][r] : b[1][r], 32, 64);
-                    ob = h ? b[1][r] : b[0][r];
-                }
-                const float ta = M == LINF ? fmaxf(oa, sa) : oa + sa;
-                const float tb = ob + sb;
-                const float v = finish<M>(ta, tb);
-                if (v <= tq && r < nvalid && qv) {
-                    const uint32_t at = atomicAdd(&cnt[q], 1u);
-                    if (at < (uint32_t)cap) cand[(size_t)q * cap + at] = make_uint2(score_key(v), (uint32_t)(rs + r));
-                }
-            }
-        }
-    }
-}
-
-template <int M>
-static void launch_m(int dpad, dim3 g, hipStream_t s, const float *base, const float *shift, const float *qry,
-                     const float *tau, int nq, long rb, long re, int nqt, int items, long item_rows, uint2 *cand,
-                     uint32_t *cnt, int cap) {
-    if (dpad <= 128 && dpad > 64)
-        scan_launch((k_valu_filter<M, 128>), g, dim3(256), 0, s, base, shift, qry, tau, nq, dpad, rb, re, nqt,
-                           items, item_rows, cand, cnt, cap);
-    else
-        scan_launch((k_valu_filter<M, 64>), g, dim3(256), 0, s, base, shift, qry, tau, nq, dpad, rb, re, nqt,
-                           items, item_rows, cand, cnt, cap);
-}
-
-void launch_valu_filter(int metric, const float *base, const float *shift, const float *qry, const float *tau,
-                        int nq, int dim, int dpad, long row_begin, long row_end, uint2 *cand, uint32_t *cnt, int cap,
-                        int grid_cap, hipStream_t s) {
-    (void)dim;
-    if (nq <= 0 || row_end <= row_begin) return;
-    const int nqt = ceil_div(nq, 256);
-    // rows per work item: small rounds are cut finer so that they still give every resident
-    // workgroup about four items
-    const long rows = row_end - row_begin;
-    long item_rows = (rows * nqt + 4L * grid_cap - 1) / (4L * grid_cap);
-    item_rows = std::min(kValuItemRowsMax, std::max(4L * kValuRows, (item_rows + kValuRows - 1) / kValuRows * kValuRows));
-    const long n_chunks = (rows + item_rows - 1) / item_rows;
-    const long items = (long)nqt * n_chunks;
-    long grid = items < grid_cap ? items : grid_cap;
-    grid = (grid + 7) / 8 * 8;
-    const dim3 g((unsigned)grid);
-    const int it = (int)items;
-    switch (metric) {
-        // squared L2 in direct form: the certified fallback of the GEMM-form L2 search
-        case L2: launch_m<L2>(dpad, g, s, base, metric == L2 ? shift : nullptr, qry, tau, nq, row_begin, row_end, nqt, it, item_rows, cand, cnt, cap); break;
-        case L1: launch_m<L1>(dpad, g, s, base, metric == L2 ? shift : nullptr, qry, tau, nq, row_begin, row_end, nqt, it, item_rows, cand, cnt, cap); break;
-        case MINK: launch_m<MINK>(dpad, g, s, base, metric == L2 ? shift : nullptr, qry, tau, nq, row_begin, row_end, nqt, it, item_rows, cand,
-                                          cnt, cap); break;
-        case LINF: launch_m<LINF>(dpad, g, s, base, metric == L2 ? shift : nullptr, qry, tau, nq, row_begin, row_end, nqt, it, item_rows, cand,
-                                          cnt, cap); break;
-        case HAMF: launch_m<HAMF>(dpad, g, s, base, metric == L2 ? shift : nullptr, qry, tau, nq, row_begin, row_end, nqt, it, item_rows, cand,
-                                          cnt, cap); break;
-        case MAHA: launch_m<MAHA>(dpad, g, s, base, metric == L2 ? shift : nullptr, qry, tau, nq, row_begin, row_end, nqt, it, item_rows, cand,
-                                          cnt, cap); break;
-        case JACC: launch_m<JACC>(dpad, g, s, base, metric == L2 ? shift : nullptr, qry, tau, nq, row_begin, row_end, nqt, it, item_rows, cand,
-                                          cnt, cap); break;
-        case HELL: launch_m<HELL>(dpad, g, s, base, metric == L2 ? shift : nullptr, qry, tau, nq, row_begin, row_end, nqt, it, item_rows, cand,
-                                          cnt, cap); break;
-        default: break;
-    }
-}
+constexpr int kValuRows = 16;  // centroid rows per LDS tile
 
 // ---------------------------------------------------------------------------------
 // k-means assignment for the non-contraction metrics (kmeans.cu:172-271): one lane per

@@ -163,7 +163,7 @@ __global__ __launch_bounds__(NT) void k_topk_merge(int k, int kc, int bufn, cons
                                                     uint32_t *__restrict__ have, float *__restrict__ tau,
                                                     uint32_t *__restrict__ flags, uint32_t *__restrict__ nflagged,
                                                     const float *__restrict__ qerr, uint32_t *__restrict__ mflag,
-                                                    uint32_t *__restrict__ mcount) {
+                                                    uint32_t *__restrict__ mcount, int drop_nan) {
     extern __shared__ u64 buf[];
     __shared__ uint32_t hist[kMergeBins];
     __shared__ uint32_t red[2 * (NT / 64)];
@@ -313,6 +313,8 @@ __global__ __launch_bounds__(NT) void k_topk_merge(int k, int kc, int bufn, cons
         }
         hn = hh;
     }
+    if (drop_nan)  // NaN scores sort behind +inf: the same count for every thread
+        while (hn > 0 && (uint32_t)(buf[hn - 1] >> 32) > score_key(INFINITY)) --hn;
     __syncthreads();
     for (uint32_t i = tid; i < hn; i += NT) tk[i] = buf[i];
     if (tid == 0) {
@@ -356,7 +358,7 @@ template <int NT>
 static void launch_merge_nt(int nq, int k, int kc, const uint2 *cand, uint32_t *cnt, int cnt_stride, int cap,
                             const uint32_t *perm,
                             unsigned long long *topk, uint32_t *have, float *tau, uint32_t *flags, uint32_t *nflagged,
-                            const float *qerr, uint32_t *mflag, uint32_t *mcount, hipStream_t s) {
+                            const float *qerr, uint32_t *mflag, uint32_t *mcount, bool drop_nan, hipStream_t s) {
     const int bufn = merge_buffer_entries(kc);
     const size_t lds = (size_t)bufn * sizeof(u64);
     static bool attr_set = false;
@@ -368,20 +370,20 @@ static void launch_merge_nt(int nq, int k, int kc, const uint2 *cand, uint32_t *
         attr_set = true;
     }
     hipLaunchKernelGGL(k_topk_merge<NT>, dim3(nq), dim3(NT), lds, s, k, kc, bufn, cand, cnt, cnt_stride, cap, perm,
-                       topk, have, tau, flags, nflagged, qerr, mflag, mcount);
+                       topk, have, tau, flags, nflagged, qerr, mflag, mcount, drop_nan ? 1 : 0);
 }
 
 void launch_topk_merge(int nq, int k, int kc, const uint2 *cand, uint32_t *cnt, int cnt_stride, int cap,
                        const uint32_t *perm, unsigned long long *topk, uint32_t *have, float *tau, uint32_t *flags,
-                       uint32_t *nflagged, const float *qerr, uint32_t *mflag, uint32_t *mcount, bool wide,
-                       hipStream_t s) {
+                       uint32_t *nflagged, const float *qerr, uint32_t *mflag, uint32_t *mcount, bool drop_nan,
+                       bool wide, hipStream_t s) {
     if (nq <= 0) return;
     if (wide)
         launch_merge_nt<1024>(nq, k, kc, cand, cnt, cnt_stride, cap, perm, topk, have, tau, flags, nflagged, qerr, mflag, mcount,
-                              s);
+                              drop_nan, s);
     else
         launch_merge_nt<256>(nq, k, kc, cand, cnt, cnt_stride, cap, perm, topk, have, tau, flags, nflagged, qerr, mflag, mcount,
-                             s);
+                             drop_nan, s);
 }
 
 __global__ void k_count_flags(const uint32_t *__restrict__ flags, int n, uint32_t *__restrict__ count) {

@@ -63,6 +63,11 @@ inline bool small_batch(int nq, int dpad, size_t n) {
     return dpad <= kSmallMaxDpad &&
            (nq <= kSmallCols || (nq <= 4 * kSmallCols && (n <= kSmallBaseRows || dpad <= 128)));
 }
+// Batches of at most kValuSmallQueries queries under the metrics that run on the vector ALUs take the
+// small-batch round plan; batches of at most kHamSmallQueries over packed codes are scanned with
+// popcounts (knn_rows.hip: the figures of both sides).
+constexpr int kValuSmallQueries = 128;
+constexpr int kHamSmallQueries = 16;
 constexpr int kRowAlign = 256;       // row counts of MFMA row operands and round boundaries
                                      // are multiples of this (the largest MFMA stage)
 
@@ -221,9 +226,19 @@ void launch_gemm_filter(int metric, bool dense, long item_rows, const float *bas
 // run's cnt[q], and the round's merge reads them there (launch_topk_merge with that stride);
 // DENSE launches write row - row_begin and leave the counts to the caller.
 constexpr int kSmallPadStride = 32, kSmallPadQueries = 4 * kSmallCols;
+static_assert(kValuSmallQueries <= kSmallPadQueries && kHamSmallQueries <= kSmallPadQueries, "a counter each");
 void launch_small_scan(int metric, bool dense, const float *base, const float *bnorm, const float *qry,
                        const float *qnorm, const float *tau, int nq, int dpad, long row_begin, long row_end,
                        long plan_rows, uint2 *cand, uint32_t *pad, int cap, int grid_cap, hipStream_t s);
+// The row-per-lane scans of the metrics on the vector ALUs, direct-form squared L2 and packed Hamming
+// (knn_rows.hip).  `base` / `qry` hold dpad floats (or code words) a row, the first dim of them used.
+// shift (may be null; squared L2): added to every base value as it is read (shifted rows that give back
+// the unshifted ones exactly).  dense: every score of the rows goes to cand[q * cap + (row - row_begin)]
+// (needs row_end - row_begin <= cap; the caller sets the counts); else query q's candidates are counted
+// on cnt[q * cnt_stride].
+void launch_row_scan(int metric, bool dense, const void *base, const float *shift, const void *qry, const float *tau,
+                     int nq, int dim, int dpad, long row_begin, long row_end, uint2 *cand, uint32_t *cnt,
+                     int cnt_stride, int cap, hipStream_t s);
 
 // Certification of the MFMA k-means assignment: each point's best score must beat its second
 // best by more than twice the point's selection error bound (err_coeff times the norms, with
@@ -261,12 +276,14 @@ void launch_topk_init(int nq, float *tau, uint32_t *have, uint32_t *cnt, uint32_
 // run's last round only): incremented once per query whose margin flag stands at the end of the
 // round, overflowed queries excepted.  wide: 1024 threads per query instead of 256 (a dense round
 // of many rows).
+// drop_nan: entries whose score is NaN leave the kept list (the VALU metrics' dense first round writes
+// every row's score; their filter rounds never pass a NaN).
 // cnt: query q's candidate count is cnt[q * cnt_stride] (1, or kSmallPadStride for a small-batch
 // FILTER round's spread counters), cleared by the merge.
 void launch_topk_merge(int nq, int k, int kc, const uint2 *cand, uint32_t *cnt, int cnt_stride, int cap,
                        const uint32_t *perm, unsigned long long *topk, uint32_t *have, float *tau, uint32_t *flags,
-                       uint32_t *nflagged, const float *qerr, uint32_t *mflag, uint32_t *mcount, bool wide,
-                       hipStream_t s);
+                       uint32_t *nflagged, const float *qerr, uint32_t *mflag, uint32_t *mcount, bool drop_nan,
+                       bool wide, hipStream_t s);
 // Where the final kernel of a search (refine or finalize) copies the two flag counters src[0..1]:
 // host = pinned host memory, or null for no copy.
 struct FlagPublish {
@@ -344,11 +361,6 @@ bool kmeans_assign_small_ok(int n, int k, int dpad, int cus);
 void launch_kmeans_assign_small(int metric, const float *pts, int dpad, int n, const float *cent, int k,
                                 int32_t *assign, float *inertia, int32_t *pos, int32_t *counts, float *devmax,
                                 hipStream_t s);
-// shift (may be null): added to every base value as the tiles are read (the direct-form pass of
-// squared L2 over shifted rows that give back the unshifted ones exactly).
-void launch_valu_filter(int metric, const float *base, const float *shift, const float *qry, const float *tau, int nq,
-                        int dim, int dpad, long row_begin, long row_end, uint2 *cand, uint32_t *cnt, int cap,
-                        int grid_cap, hipStream_t s);
 // Fills count floats (32-bit words) with v.  Kernels rather than hipMemsetAsync, so a caller may
 // capture the engines' work in a HIP graph.
 void launch_fill(float *p, size_t count, float v, hipStream_t s);
