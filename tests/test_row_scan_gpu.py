@@ -79,3 +79,18 @@ def test_hamming_small_batches(vh, words, n, k):
         i2, d2, _ = eng.search_batch_arrays(q[:nq], k)
         np.testing.assert_array_equal(i2[:, :kk], ids[:nq, :kk])
         np.testing.assert_array_equal(d2[:, :kk], dist[:nq, :kk])
+
+
+@pytest.mark.parametrize("words", [2, 8, 32])
+@pytest.mark.parametrize("nq", [17, 128, 129, 256])
+def test_hamming_mid_batches(vh, monkeypatch, words, nq):
+    """Mid-size batches on the fp4 matrix cores take the small-batch round plan (dense rounds cut into
+    512-row items); the popcount batch kernel has the growing plan and is the reference here."""
+    rng = np.random.default_rng(words + nq)
+    codes = rng.integers(0, 1 << 32, (150_001, words), dtype=np.uint64).astype(np.uint32)
+    q = rng.integers(0, 1 << 32, (nq, words), dtype=np.uint64).astype(np.uint32)
+    ids, dist, _ = vh.HammingKnnEngine(codes).search_batch_arrays(q, 30)
+    monkeypatch.setenv("VHIP_HAMMING_KERNEL", "popcount")
+    i2, d2, _ = vh.HammingKnnEngine(codes).search_batch_arrays(q, 30)
+    np.testing.assert_array_equal(ids, i2)
+    np.testing.assert_array_equal(dist, d2)

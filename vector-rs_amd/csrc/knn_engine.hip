@@ -360,8 +360,11 @@ static bool small_scan_run(const vhip_knn *E, size_t nq, bool direct) {
     if (E->metric == HAMMING_PACKED) return E->ham_small && nq <= (size_t)kHamSmallQueries;
     return nq <= (size_t)kValuSmallQueries;
 }
-// ... which run on the small-batch round plan.
-static bool small_plan(const vhip_knn *E, size_t nq, bool direct) { return small_scan_run(E, nq, direct); }
+// Whether it takes the small-batch round plan: with those scans, and for batches of up to
+// kHamSmallRounds queries on the fp4 matrix cores.
+static bool small_plan(const vhip_knn *E, size_t nq, bool direct) {
+    return small_scan_run(E, nq, direct) || (E->ham8 && nq <= (size_t)kHamSmallRounds);
+}
 
 // The candidate count a run starts from: the first round's rows when that round is dense (every
 // score is written), else 0.
@@ -433,8 +436,11 @@ static int run_rounds(vhip_knn *E, const QueryRows &Q, int nq, int k, int kc, in
                 launch_ham_mfma_wide(witem, E->base8.as<int8_t>(), B.q8, (int)E->dpad, B.tau, nq, rb, re, B.cand,
                                      B.cnt, cap, E->grid_cap, s);
             } else {
+                // a dense round has no slots to spare or flush, so its items are one 512-row stage: as one
+                // item an 8,192-row round ran on one workgroup per 128 queries (4M x 256 bits, 17 queries:
+                // 278 us a search against 167)
                 const long hitem =
-                    dense ? re - rb
+                    dense ? std::min<long>(re - rb, 512)
                           : balanced_item(std::min<long>(32768, rd.slot_rows), re - rb, ceil_div(nq, kTileCols),
                                           E->grid_cap / 2, 512);
                 launch_ham_mfma(dense, hitem, E->base8.as<int8_t>(), B.q8, (int)E->dpad, B.tau, nq, rb, re, B.cand,

@@ -68,6 +68,11 @@ inline bool small_batch(int nq, int dpad, size_t n) {
 // popcounts (knn_rows.hip: the figures of both sides).
 constexpr int kValuSmallQueries = 128;
 constexpr int kHamSmallQueries = 16;
+// Packed Hamming on the fp4 matrix cores takes the small-batch round plan (three rounds at 4M rows where
+// the growing plan has eight) up to this many queries.  Past that the merges of its 8,192-row first round
+// cost more than the rounds saved: 4M x 256 bits, k = 10: 17 queries 231 -> 167 us, 128 270 -> 207, 256
+// 300 -> 263, but 512 422 -> 407 and 1,024 627 -> 672; 1M x 64 bits: 256 191 -> 191, 512 225 -> 293.
+constexpr int kHamSmallRounds = 256;
 constexpr int kRowAlign = 256;       // row counts of MFMA row operands and round boundaries
                                      // are multiples of this (the largest MFMA stage)
 
