@@ -1,0 +1,87 @@
+"""PQ training and encoding of narrow sub-vectors (pq_train.hip), all sub-spaces in one launch.
+
+Training under squared L2 is held to the general k-means engine run on each sub-space by itself, which
+it replaces there: on whole-number data whose sums stay exact, the codebooks agree to the last bits of
+the centroid division.  Encoding is held to the oracle's argmin in every metric."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def vh():
+    import vector_hip
+
+    assert vector_hip.CudaDeviceContext.device_count() >= 1
+    return vector_hip
+
+
+# padded widths 4, 8, 16, 32 and their edges, one and several workgroups, odd cluster counts, n < ks
+@pytest.mark.parametrize("n,ds,m,ks,iters", [(1, 1, 1, 4, 2), (255, 3, 2, 7, 3), (513, 4, 1, 1, 2), (3000, 5, 3, 256, 4),
+                                             (20_001, 8, 4, 255, 3), (5000, 9, 2, 64, 5), (70_000, 16, 2, 256, 3),
+                                             (4097, 17, 2, 33, 4), (9000, 32, 3, 256, 3), (100, 32, 2, 256, 0)])
+@pytest.mark.parametrize("given", [True, False])
+def test_train_equals_the_general_engine(vh, n, ds, m, ks, iters, given):
+    rng = np.random.default_rng(n + ds)
+    x = rng.integers(-60, 60, (n, m * ds)).astype(np.float32)
+    ek = min(ks, n)
+    init = None
+    if given:
+        init = np.zeros((m, ks, ds), np.float32)
+        for j in range(m):
+            init[j, :ek] = x[rng.permutation(n)[:ek], j * ds:(j + 1) * ds]
+    pq = vh.ProductQuantizer.train(x, m * ds, m, ks, iters, -1.0, seed=11, init_codebooks=init)
+    got = pq.codebooks.reshape(m, ks, ds)
+    for j in range(m):
+        sub = np.ascontiguousarray(x[:, j * ds:(j + 1) * ds])
+        st = vh.KMeansState(sub)
+        c, _, _ = st.fit(ks, iters, -1.0, init=None if init is None else init[j, :ek], init_mode=vh.INIT_SHUFFLE,
+                         seed=11 + 1 + j)
+        np.testing.assert_allclose(got[j, :ek], c, rtol=1e-6, atol=1e-6)
+        assert not got[j, ek:].any()
+
+
+def test_sub_spaces_stop_by_themselves(vh):
+    """With a tolerance each sub-space stops at its own iteration: the first is at a fixed point from the
+    start (one iteration), the second is not."""
+    rng = np.random.default_rng(5)
+    a = np.repeat(np.array([[0, 0], [100, 0], [0, 100], [100, 100]], np.float32), 500, 0)
+    b = rng.integers(0, 1000, (2000, 2)).astype(np.float32)
+    x = np.concatenate([a, b], 1)
+    init = np.zeros((2, 4, 2), np.float32)
+    init[0], init[1] = a[::500], b[:4]
+    got = vh.ProductQuantizer.train(x, 4, 2, 4, 40, 1e-4, init_codebooks=init).codebooks.reshape(2, 4, 2)
+    np.testing.assert_array_equal(got[0], a[::500])
+    c, _, r = vh.KMeansState(np.ascontiguousarray(b)).fit(4, 40, 1e-4, init=b[:4])
+    assert 1 < r[2] < 40
+    np.testing.assert_allclose(got[1], c, rtol=1e-6)
+
+
+def test_infinite_values_are_refused(vh):
+    x = np.zeros((300, 8), np.float32)
+    x[7, 5] = np.inf
+    with pytest.raises(vh.InvalidConfig):
+        vh.ProductQuantizer.train(x, 8, 2, 4, 2, -1.0)
+
+
+@pytest.mark.parametrize("metric", ["l2", "dot", "cosine", "l1", "minkowski", "linf", "hamming", "mahalanobis",
+                                    "jaccard", "hellinger"])
+@pytest.mark.parametrize("n,ds,m,ks", [(1, 1, 3, 2), (257, 6, 2, 255), (513, 16, 1, 256), (1000, 31, 2, 3)])
+def test_encode_narrow(vh, oracle, metric, n, ds, m, ks):
+    rng = np.random.default_rng(ds * 100 + ks)
+    codes = {"l2": 0, "dot": 1, "cosine": 2, "l1": 3, "minkowski": 4, "linf": 5, "hamming": 6, "mahalanobis": 7,
+             "jaccard": 8, "hellinger": 9}
+    cb = rng.integers(-5, 6, (m, ks, ds)).astype(np.float32)
+    x = rng.integers(-5, 6, (n, m * ds)).astype(np.float32)
+    pq = vh.ProductQuantizer(m * ds, m, ks, cb)
+    got = pq.encode_batch(x, vh.DistanceMetric(codes[metric]))
+    for j in range(m):
+        sub, c = np.ascontiguousarray(x[:, j * ds:(j + 1) * ds]), cb[j]
+        d = np.stack([oracle.distance_rows(metric, sub, np.repeat(c[t:t + 1], n, 0)) for t in range(ks)], 1)
+        best = d.max(1) if metric in ("dot", "cosine") else d.min(1)
+        mine = d[np.arange(n), got[:, j]]
+        np.testing.assert_allclose(mine, best, rtol=2e-6, atol=2e-6)
+        if metric in ("l2", "dot", "l1", "linf", "hamming"):  # exact values: the lowest index among equals
+            first = (d.argmax(1) if metric == "dot" else d.argmin(1))
+            np.testing.assert_array_equal(got[:, j], first)

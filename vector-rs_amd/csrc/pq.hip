@@ -1,9 +1,11 @@
 // pq.hip -- product quantization and the IVF-PQ index on one GPU behind the C ABI.
 //
 // ProductQuantizer (vector-index/src/ivf/pq.rs) and IvfPqIndex (ivf/mod.rs):
-//  * train: one k-means per sub-space (pq.rs:53-107) on the GPU k-means engine;
-//  * encode (pq.rs:178-214): k_pq_encode, one thread per (vector, sub-space), the strict-compare
-//    argmin of find_nearest_centroid (ivf/kmeans.rs:262-309) over the sub-space's codebook in LDS;
+//  * train: one k-means per sub-space (pq.rs:53-107), all at once under squared L2 (pq_train.hip), else
+//    on the GPU k-means engine;
+//  * encode (pq.rs:178-214): the strict-compare argmin of find_nearest_centroid
+//    (ivf/kmeans.rs:262-309), in pq_train.hip for sub-vectors of at most 32 dimensions, else
+//    k_pq_encode, one thread per (vector, sub-space) with the sub-space's codebook in LDS;
 //  * compute_adc_lut (pq.rs:233-266): k_pq_lut, one thread per table entry;
 //  * search (ivf/mod.rs:256-345): coarse probe through a kNN engine over the coarse centroids
 //    (k = nprobe, best first), then the fused ADC scan k_ivfpq_scan (pq_scan.h).
@@ -20,8 +22,7 @@
 namespace vh {
 namespace {
 
-// ---- encode -------------------------------------------------------------------------------
-constexpr int kEncRegDims = 32;          // sub-vector floats held in registers
+// ---- encode, sub-vectors of more than 32 dimensions (shorter ones: pq_train.hip) -----------
 constexpr int kEncLdsFloats = 16384;     // codebooks up to 64 KB are staged in LDS
 
 // Block (x, m): 256 vectors, sub-space m.  Codebook m in LDS when it fits (cb_lds), else read
@@ -44,32 +45,14 @@ __global__ __launch_bounds__(256) void k_pq_encode(const float *__restrict__ x, 
     constexpr bool hib = hib_metric(MT);
     float best = hib ? -INFINITY : INFINITY;
     int bi = 0;
-    if (ds <= kEncRegDims) {
-        float xr[kEncRegDims];
-#pragma unroll
-        for (int d = 0; d < kEncRegDims; ++d) xr[d] = d < ds ? xs[d] : 0.0f;
-        for (int j = 0; j < ks; ++j) {
-            Acc<MT> acc;
-            const float *c = cw + j * ds;
-#pragma unroll
-            for (int d = 0; d < kEncRegDims; ++d)
-                if (d < ds) acc.step(xr[d], c[d]);
-            const float v = acc.finish();
-            if (hib ? v > best : v < best) {
-                best = v;
-                bi = j;
-            }
-        }
-    } else {
-        for (int j = 0; j < ks; ++j) {
-            Acc<MT> acc;
-            const float *c = cw + j * ds;
-            for (int d = 0; d < ds; ++d) acc.step(xs[d], c[d]);
-            const float v = acc.finish();
-            if (hib ? v > best : v < best) {
-                best = v;
-                bi = j;
-            }
+    for (int j = 0; j < ks; ++j) {
+        Acc<MT> acc;
+        const float *c = cw + j * ds;
+        for (int d = 0; d < ds; ++d) acc.step(xs[d], c[d]);
+        const float v = acc.finish();
+        if (hib ? v > best : v < best) {
+            best = v;
+            bi = j;
         }
     }
     codes[i * m_sub + m] = (uint8_t)bi;
@@ -136,6 +119,13 @@ static int scan_pg(size_t dim, size_t m_sub, size_t ks, size_t k) {
     return 1;
 }
 
+// pq_train.hip: sub-vectors of at most 32 dimensions
+bool pq_narrow(size_t ds);
+int pq_encode_narrow(const float *d_x, size_t n, size_t dim, size_t m_sub, size_t ks, int metric, const float *codebooks,
+                     int dev, uint8_t *d_codes, DevBuf &cent, hipStream_t s);
+int pq_train_batched(int ordinal, const float *data, size_t n, size_t dim, size_t m_sub, size_t ks, size_t max_iters,
+                     float tol, const float *init_codebooks, uint64_t seed, float *out_codebooks);
+
 }  // namespace vh
 
 using namespace vh;
@@ -195,7 +185,7 @@ static int upload(DevBuf &b, int dev, const void *src, size_t bytes, hipStream_t
     return VHIP_OK;
 }
 
-static int pq_encode_dev(int dev, const float *d_x, size_t n, size_t dim, size_t m_sub, size_t ks, int metric,
+static int pq_encode_dev(const float *d_x, size_t n, size_t dim, size_t m_sub, size_t ks, int metric,
                          const float *d_cb, uint8_t *d_codes, hipStream_t s) {
     if (n == 0) return VHIP_OK;
     const size_t ds = dim / m_sub;
@@ -208,7 +198,6 @@ static int pq_encode_dev(int dev, const float *d_x, size_t n, size_t dim, size_t
     VH_METRIC_SWITCH(metric, VH_ENC)
 #undef VH_ENC
     VH_HIP(hipGetLastError());
-    (void)dev;
     return VHIP_OK;
 }
 
@@ -645,6 +634,10 @@ int vhip_pq_train(int ordinal, const float *data, size_t n, size_t dim, size_t m
     std::fill(out_codebooks, out_codebooks + m_sub * ks * ds, 0.0f);  // pq.rs:84-88 zero padding
     if (n == 0) return VHIP_OK;
     if (!data) return set_error(VHIP_ERR_INVALID_CONFIG, "data is null");
+    // squared L2 over narrow sub-vectors: all sub-spaces at once (65,536 x 128, 8 sub-spaces of 256, 10
+    // iterations: 21 -> 3.3 ms); else one general k-means after another
+    if (metric == L2 && pq_narrow(ds))
+        return pq_train_batched(ordinal, data, n, dim, m_sub, ks, max_iters, tol, init_codebooks, seed, out_codebooks);
     std::vector<float> sub(n * ds);
     for (size_t m = 0; m < m_sub; ++m) {
         for (size_t i = 0; i < n; ++i)  // pq.rs:69-74: sub-vector m of every sample
@@ -668,14 +661,18 @@ int vhip_pq_encode(int ordinal, const float *codebooks, size_t dim, size_t m_sub
     VH_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     std::unique_ptr<ihipStream_t, hipError_t (*)(hipStream_t)> hold(s, hipStreamDestroy);
     PinnedStager st;
-    VH_CHECK(st.init(ordinal));
+    st.dev = ordinal;
     DevBuf x, cb, codes;
     VH_CHECK(x.ensure(ordinal, n * dim * 4));
-    VH_CHECK(st.h2d(x.p, data, n * dim * 4, s));
-    VH_CHECK(upload(cb, ordinal, codebooks, m_sub * ks * (dim / m_sub) * 4, s));
+    VH_CHECK(st.h2d_once(x.p, data, n * dim * 4, s));
     VH_CHECK(codes.ensure(ordinal, n * m_sub));
-    VH_CHECK(pq_encode_dev(ordinal, x.as<float>(), n, dim, m_sub, ks, metric, cb.as<float>(), codes.as<uint8_t>(), s));
-    VH_CHECK(st.d2h(out_codes, codes.p, n * m_sub, s));
+    if (pq_narrow(dim / m_sub)) {
+        VH_CHECK(pq_encode_narrow(x.as<float>(), n, dim, m_sub, ks, metric, codebooks, ordinal, codes.as<uint8_t>(), cb, s));
+    } else {
+        VH_CHECK(upload(cb, ordinal, codebooks, m_sub * ks * (dim / m_sub) * 4, s));
+        VH_CHECK(pq_encode_dev(x.as<float>(), n, dim, m_sub, ks, metric, cb.as<float>(), codes.as<uint8_t>(), s));
+    }
+    VH_HIP(hipMemcpyAsync(out_codes, codes.p, n * m_sub, hipMemcpyDeviceToHost, s));
     VH_HIP(hipStreamSynchronize(s));
     return VHIP_OK;
 }

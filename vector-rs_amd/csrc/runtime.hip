@@ -188,6 +188,13 @@ int PinnedStager::h2d(void *dst, const void *src, size_t bytes, hipStream_t s) {
     return VHIP_OK;
 }
 
+int PinnedStager::h2d_once(void *dst, const void *src, size_t bytes, hipStream_t s) {
+    if (bytes > kOneOff) return h2d(dst, src, bytes, s);
+    VH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
+    VH_HIP(hipStreamSynchronize(s));
+    return VHIP_OK;
+}
+
 int PinnedStager::d2h(void *dst, const void *src, size_t bytes, hipStream_t s) {
     VH_CHECK(init(dev < 0 ? 0 : dev));
     size_t off = 0;
