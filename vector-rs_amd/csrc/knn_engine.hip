@@ -102,8 +102,8 @@ struct vhip_knn {
 namespace vh {
 
 // Search rounds.  Round 0 scores rows [0, b0) with b0 about 20 k, the first 256-row multiple
-// at or above it (all rows when the base has at most max(2048, 32 k)): for the GEMM metrics
-// densely (every score written, no atomics), for the others through the filter with tau = +inf.
+// at or above it and at least kFirstRows (all rows when the base has at most max(2048, 32 k)), densely
+// (every score written, no atomics); the popcount batch kernel alone filters it with tau = +inf.
 // Every later round covers about 4 times the rows seen so far (the growth factor, see
 // kRoundGrowth) and keeps only rows scoring <= tau, the k-th best so far.  Because the base rows
 // are in a pseudo-random order, round i passes about k * (rows_i / seen_i) ~ 3 k candidates per
@@ -133,17 +133,20 @@ constexpr int kRoundGrowth = 4;
 // k = 100 three rounds.)  A larger first round costs more in its merge (32,768 rows: 27 us against
 // about 12) than the fewer passes save.
 constexpr size_t kSmallDenseRows = 8192;
-// Batches the row-per-lane scan serves above that size start with this many dense rows at least: the
-// scan's small rounds cost about as much as its launches and merges, whatever their rows (L1 500k x 128,
-// 700 queries 1906 -> 1862 us, 4,096 queries 10528 -> 10163; L-inf 150,001 x 100, 700 queries 625 -> 610).
-constexpr size_t kRowScanFirst = 2048;
+// A dense first round has at least this many rows: a small round costs about as much as its launch and
+// merge, whatever its rows, and 2,048 candidates a query is the lists' least capacity anyway.  Against a
+// start of 256 rows (512 at k = 20), whole searches: L1 500k x 128, 4,096 queries 10528 -> 10163 us; dot
+// 200,003 x 300, k = 20, 129 queries 346 -> 309, 1,000 1171 -> 1136; cosine 20,000 x 64, 1,000 queries
+// 170 -> 128, 8,000 486 -> 433; squared L2 1M x 128, 8,000 queries 14901 -> 14835; fp4 Hamming 4M x 256
+// bits, 512 queries 426 -> 397, 10,000 3793 -> 3776 (100k x 256: 10,000 queries 516 -> 525).
+constexpr size_t kFirstRows = 2048;
 
-static std::vector<Round> plan_rounds(size_t n, size_t k, bool dense0, int dpad, int growth, bool small = false,
-                                      size_t first = 256) {
+static std::vector<Round> plan_rounds(size_t n, size_t k, bool dense0, int dpad, int growth,
+                                      bool small = false) {
     std::vector<Round> r;
     if (n == 0) return r;
     const size_t kk = std::max<size_t>(k, 1);
-    size_t b0 = std::min(n, round_up(std::max<size_t>(first, 20 * kk), kRowAlign));
+    size_t b0 = std::min(n, round_up(std::max<size_t>(dense0 ? kFirstRows : 256, 20 * kk), kRowAlign));
     // A base within the candidate capacity's floor (round_cap) is scored in one dense round: its
     // later rounds would cost more launches than rows (the IVF coarse probe: 1,024 centroids).
     if (n <= std::max<size_t>(2048, 32 * kk)) b0 = n;
@@ -374,8 +377,7 @@ static uint32_t first_count(const std::vector<Round> &rounds) {
 // The rounds of a run.  The first is dense on every path but the popcount batch kernel's.
 static std::vector<Round> run_plan(const vhip_knn *E, int k, bool small, long max_round_rows) {
     const bool dense0 = E->metric != HAMMING_PACKED || E->ham8 || small;
-    const size_t first = is_gemm_metric(E->metric) || E->metric == HAMMING_PACKED ? 256 : kRowScanFirst;
-    return split_rounds(plan_rounds(E->n, (size_t)k, dense0, (int)E->dpad, kRoundGrowth, small, first), max_round_rows);
+    return split_rounds(plan_rounds(E->n, (size_t)k, dense0, (int)E->dpad, kRoundGrowth, small), max_round_rows);
 }
 
 // Runs all rounds for nq prepared queries; results stay in B.topk (row stride kc) / B.have.
@@ -480,9 +482,8 @@ static int run_rounds(vhip_knn *E, const QueryRows &Q, int nq, int k, int kc, in
 // plan.
 static int full_cap(const vhip_knn *E, size_t k) {
     long big = k;
-    for (int sm = 0; sm < 3; ++sm)
-        for (const Round &rd : plan_rounds(E->n, k, true, (int)E->dpad, kRoundGrowth, sm == 1,
-                                           sm == 2 ? kRowScanFirst : 256))
+    for (int v = 0; v < 4; ++v)
+        for (const Round &rd : plan_rounds(E->n, k, (v & 1) != 0, (int)E->dpad, kRoundGrowth, (v & 2) != 0))
             big = std::max(big, rd.re - rd.rb);
     return (int)round_up((size_t)big, kRowAlign);
 }

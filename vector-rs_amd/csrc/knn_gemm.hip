@@ -1450,7 +1450,11 @@ __global__ __launch_bounds__(512, 1) void k_mfma_hs(ScanArgs a) {
 }
 
 // =========================================================================================
-// Narrow resident-tile kernel (kNN search at dpad a multiple of 128 from 256 to 896).  A work item is
+// Narrow resident-tile kernel (kNN search at dpad from 160 to 896, every multiple of 32).  Widths that are
+// no multiple of 128 ran on k_mfma_stream, which passes both operands through LDS with a barrier per
+// K-chunk: dot 200,003 x 300, k = 20: 1,000 queries 1730 -> 1140 us, 8,000 9262 -> 8081 (96 TFLOP/s of
+// 153 -> 119); squared L2 150,000 x 784: 1,000 queries 3332 -> 2050, 8,000 19985 -> 14707; cosine 200,000 x
+// 200: 1,000 queries 1230 -> 895 (starts of kFirstRows included in the first two).  A work item is
 // kNtCols = 32 query columns, whose 32 x dpad tile stays resident in LDS (96 KB at dpad 768), x
 // item_rows base rows in stages of 512: each of the 8 waves streams its own 64 rows of A from L2
 // into registers two K-chunks ahead and computes its 64 x 32 block in two
@@ -1488,12 +1492,13 @@ __global__ __launch_bounds__(512, 1) void k_mfma_nt(ScanArgs a) {
         const int pch = (NK % 2 == 0) ? (kc ^ (r & 1)) : kc;
         return r * (8 * NK) + pch * 8 + (c4 ^ ((r >> 1) & 7));
     };
+    // (an odd NK leaves half of the threads without a piece in the last pass: they repeat the tile's last)
     auto fill_b = [&](int c0) {
-        constexpr int PER = TC * 8 * NK / 512;
+        constexpr int PIECES = TC * 8 * NK, PER = (PIECES + 511) / 512;
         floatx4 rq[PER];
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
-            const int f = tid + 512 * i;
+            const int f = min(tid + 512 * i, PIECES - 1);
             const int r = f / (8 * NK), rem = f % (8 * NK);
             rq[i] = *(const floatx4 *)(a.B + (long)(c0 + r) * D + 4 * rem);
         }
@@ -1503,7 +1508,7 @@ __global__ __launch_bounds__(512, 1) void k_mfma_nt(ScanArgs a) {
         }
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
-            const int f = tid + 512 * i;
+            const int f = min(tid + 512 * i, PIECES - 1);
             const int r = f / (8 * NK), rem = f % (8 * NK);
             sB[bidx_kc(r, rem >> 3, rem & 7)] = rq[i];
         }
@@ -1699,20 +1704,20 @@ static void launch_scan(const ScanArgs &a, int grid_cap, hipStream_t s) {
             case 3: scan_launch((k_mfma_hs<MODE, M, 3>), g, b, 0, s, a); break;
             default: scan_launch((k_mfma_hs<MODE, M, 4>), g, b, 0, s, a); break;
         }
-    } else if (nk % 4 == 0) {
+    } else if (MODE != kAssign && gemm_narrow(a.dpad)) {
         const dim3 g(grid_for(a.n_items, cus));
         if constexpr (MODE != kAssign) {
-            switch (gemm_filter_cols(a.dpad) == kNtCols ? nk : 0) {  // the narrow-tile instantiations
-                case 8: scan_launch((k_mfma_nt<MODE, M, 8>), g, dim3(512), 0, s, a); return;
-                case 12: scan_launch((k_mfma_nt<MODE, M, 12>), g, dim3(512), 0, s, a); return;
-                case 16: scan_launch((k_mfma_nt<MODE, M, 16>), g, dim3(512), 0, s, a); return;
-                case 20: scan_launch((k_mfma_nt<MODE, M, 20>), g, dim3(512), 0, s, a); return;
-                case 24: scan_launch((k_mfma_nt<MODE, M, 24>), g, dim3(512), 0, s, a); return;
-                case 28: scan_launch((k_mfma_nt<MODE, M, 28>), g, dim3(512), 0, s, a); return;
+            switch (nk) {  // the narrow-tile instantiations: every row width gemm_narrow() takes
+#define VH_NT(NK) case NK: scan_launch((k_mfma_nt<MODE, M, NK>), g, dim3(512), 0, s, a); return;
+                VH_NT(5) VH_NT(6) VH_NT(7) VH_NT(8) VH_NT(9) VH_NT(10) VH_NT(11) VH_NT(12)
+                VH_NT(13) VH_NT(14) VH_NT(15) VH_NT(16) VH_NT(17) VH_NT(18) VH_NT(19) VH_NT(20)
+                VH_NT(21) VH_NT(22) VH_NT(23) VH_NT(24) VH_NT(25) VH_NT(26) VH_NT(27) VH_NT(28)
+#undef VH_NT
                 default: break;
             }
         }
-        scan_launch((k_mfma_pnl<MODE, M>), g, dim3(512), 0, s, a);
+    } else if (nk % 4 == 0) {
+        scan_launch((k_mfma_pnl<MODE, M>), dim3(grid_for(a.n_items, cus)), dim3(512), 0, s, a);
     } else {
         const dim3 g(grid_for(a.n_items, 2 * cus)), b(256);
         scan_launch((k_mfma_stream<MODE, M>), g, b, 0, s, a);

@@ -41,9 +41,9 @@ constexpr int kKChunk = 32;          // K (dimension) chunk of the MFMA tiles
 constexpr int kTileCols = 128;       // queries (or k-means points) per MFMA work item
 constexpr int kNtCols = 32;          // queries per work item of the narrow resident-tile kernel
 // Query columns per work item of the MFMA search kernel that serves rows of dpad floats: the
-// narrow resident-tile kernel takes dpad a multiple of 128 from 256 to 896 (its 32 x dpad query
-// tile stays in LDS), the others kTileCols.
-inline bool gemm_narrow(int dpad) { return dpad % 128 == 0 && dpad >= 256 && dpad <= 896; }
+// narrow resident-tile kernel takes dpad from 160 to 896 (its 32 x dpad query tile stays in LDS), the
+// others kTileCols.
+inline bool gemm_narrow(int dpad) { return dpad > 128 && dpad <= 896; }
 inline int gemm_filter_cols(int dpad) { return gemm_narrow(dpad) ? kNtCols : kTileCols; }
 // LDS candidate slots of the MFMA search kernel that serves rows of dpad floats
 inline int gemm_slots(int dpad) {
