@@ -27,9 +27,9 @@ def vh():
     return vector_hip
 
 
-def _skewed_parts(rng, dim, nlist, n, empty=(), integer=False):
+def _skewed_parts(rng, dim, nlist, n, empty=(), integer=False, m_sub=16):
     """Lists of very different sizes (a few hold most rows), some empty."""
-    m_sub, ks, ds = 16, 256, dim // 16
+    ks, ds = 256, dim // m_sub
     if integer:
         coarse = rng.integers(-4, 5, (nlist, dim)).astype(np.float32)
         cb = rng.integers(-2, 3, m_sub * ks * ds).astype(np.float32)
@@ -140,3 +140,15 @@ def test_batch_of_several_chunks(vh):
     head = ix.search_batch_arrays(qs[:40_000], 10, 64)
     tail = ix.search_batch_arrays(qs[40_000:], 10, 64)
     _assert_same(whole, tuple(np.concatenate([h, t]) for h, t in zip(head, tail)))
+
+
+@pytest.mark.parametrize("metric", ["L2Squared", "DotProduct", "CosineSimilarity"])
+@pytest.mark.parametrize("dim,k,nprobe,nq", [(32, 10, 8, 1024), (64, 1, 1, 1500), (128, 16, 64, 1100), (128, 10, 3, 2001),
+                                             (64, 48, 16, 4100), (128, 10, 8, 1023)])
+def test_eight_byte_rows_match_query_major(vh, metric, dim, k, nprobe, nq):
+    """8-byte code rows at each sub-vector width, on both sides of the batch sizes that choose the path."""
+    rng = np.random.default_rng(dim + 31 * k + nprobe)
+    parts = _skewed_parts(rng, dim, 64, 50_000, empty=(5, 17, 40), m_sub=8)
+    ix = _index(vh, parts, dim, 8, 256, vh.DistanceMetric[metric])
+    a, b = _both_paths(ix, rng.standard_normal((nq, dim)).astype(np.float32), k, nprobe)
+    _assert_same(a, b)

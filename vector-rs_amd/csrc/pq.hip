@@ -459,14 +459,24 @@ void ivfpq_list_plan(const uint32_t *probes, int nq, int nprobe, int nlist, cons
                        kListQb, n_items, items, item_pairs);
 }
 
-// The list-major search applies to 16-byte code rows of 256 sub-centroids with the register-held
-// codebook (ds 4 or 8) and k <= kListMaxK; VHIP_IVFPQ_SCAN=query forces the query-major kernel.
-static bool list_path(const vhip_ivfpq *X, size_t k, size_t np) {
+// The list-major search applies to code rows of 16 or 8 bytes of 256 sub-centroids with the register-held
+// codebook (ds 4 or 8, with 8-byte rows also 16) and k <= kListMaxK; VHIP_IVFPQ_SCAN=query forces the
+// query-major kernel.  With 8-byte rows a table holds half as much, so the query-major kernel, one
+// workgroup a query and 512 resident, keeps up until they have run twice over (later for a larger k, whose
+// merge of nprobe k keys costs the list-major search more).  Whole searches, query-major / list-major us:
+//   400k x 128, nlist 512, nprobe 16, k = 10:  500 queries 162 / 216,  2,000 405 / 373,  8,000 1374 / 995
+//   400k x 32, the same:                       500 151 / 182,          2,000 395 / 310,  8,000 1374 / 820
+//   300k x 64, nlist 512, nprobe 4, k = 1:     500 107 / 134,          2,000 232 / 180,  8,000 734 / 352
+//   100k x 128, nlist 64, nprobe 8, k = 40:    500 156 / 243,          2,000 389 / 447,  8,000 1326 / 1204
+constexpr size_t kListMinQueries8 = 1024, kListMinQueries8LargeK = 4096, kListSmallK8 = 16;
+static bool list_path(const vhip_ivfpq *X, size_t nq, size_t k, size_t np) {
     if (const char *e = std::getenv("VHIP_IVFPQ_SCAN"))
         if (std::strcmp(e, "query") == 0) return false;
-    return X->reg && X->ks == 256 && X->m_sub == 16 && (X->ds == 4 || X->ds == 8) && k >= 1 &&
-           k <= (size_t)kListMaxK && np * k <= (size_t)kListMaxMerge &&
-           sizeof(ListLds) <= X->lds_limit;
+    const bool shape16 = X->m_sub == 16 && (X->ds == 4 || X->ds == 8);
+    const bool shape8 = X->m_sub == 8 && (X->ds == 4 || X->ds == 8 || X->ds == 16) &&
+                        nq >= (k <= kListSmallK8 ? kListMinQueries8 : kListMinQueries8LargeK);
+    return X->reg && X->ks == 256 && (shape16 || shape8) && k >= 1 && k <= (size_t)kListMaxK &&
+           np * k <= (size_t)kListMaxMerge && sizeof(ListLds<16>) <= X->lds_limit;
 }
 
 // (query, probe) pairs of one search chunk: pair ids are 32-bit (q * nprobe + p) and the plan's
@@ -479,7 +489,7 @@ static int ivfpq_search_chunk(vhip_ivfpq *X, const float *d_q, size_t nq, size_t
     hipStream_t s = X->stream;
     VH_CHECK(X->d_pid.ensure(X->dev, nq * np * 4));
     VH_CHECK(X->d_pdist.ensure(X->dev, nq * np * 4));
-    const bool lists = list_path(X, k, np);
+    const bool lists = list_path(X, nq, k, np);
     if (lists) {
         // the plan's buffers, cleared on this stream while the probe runs on the probe engine's
         const size_t total = nq * np;

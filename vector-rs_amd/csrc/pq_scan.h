@@ -632,8 +632,9 @@ __global__ __launch_bounds__(kScanThreads) void k_ivfpq_scan(ScanArgs A) {
 
 // LDS of k_ivfpq_lists, the tables first: they lie at LDS offset 0, so a lookup takes its
 // sub-space's table address as the instruction's offset.
+template <int M>
 struct ListLds {
-    float4 lut[16 * 256];                                  // entry (m, e): the four pairs' values
+    float4 lut[M * 256];                                   // entry (m, e): the four pairs' values
     unsigned long long cand[kListQb * kListCapw];          // candidates (residuals before the scan)
     float score[2][kListQb][kListChunkRows];               // per chunk parity: each pair's row scores
     uint32_t item;
@@ -654,14 +655,38 @@ __device__ __forceinline__ uint32_t byte_x16(uint32_t w) {
     return a;
 }
 
-// The four pairs' scores of one code row (16 bytes) against the float4 tables at LDS offset 0:
-// per pair, sum over words h of ((d0 + d1) + (d2 + d3)).
-__device__ __forceinline__ float4 row_score4(const float4 *lut, uint4 w) {
+// A code row of W words.
+template <int W>
+struct CodeRow {
+    uint32_t w[W];
+};
+template <int W>
+__device__ __forceinline__ CodeRow<W> load_code_row(const uint8_t *p) {
+    CodeRow<W> r;
+    if constexpr (W == 4) {
+        const uint4 v = *reinterpret_cast<const uint4 *>(p);
+        r.w[0] = v.x;
+        r.w[1] = v.y;
+        r.w[2] = v.z;
+        r.w[3] = v.w;
+    } else {
+        static_assert(W == 2, "8- or 16-byte rows");
+        const uint2 v = *reinterpret_cast<const uint2 *>(p);
+        r.w[0] = v.x;
+        r.w[1] = v.y;
+    }
+    return r;
+}
+
+// The four pairs' scores of one code row against the float4 tables at LDS offset 0: per pair, sum over
+// words h of ((d0 + d1) + (d2 + d3)).
+template <int W>
+__device__ __forceinline__ float4 row_score4(const float4 *lut, const CodeRow<W> &w) {
     const char *base = reinterpret_cast<const char *>(lut);
-    const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
+    const uint32_t(&ww)[W] = w.w;
     float4 total = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
-    for (int h = 0; h < 4; ++h) {
+    for (int h = 0; h < W; ++h) {
         const char *L = base + 4 * h * 4096;
         const float4 d0 = *reinterpret_cast<const float4 *>(L + byte_x16<0>(ww[h]));
         const float4 d1 = *reinterpret_cast<const float4 *>(L + 4096 + byte_x16<1>(ww[h]));
@@ -675,12 +700,12 @@ __device__ __forceinline__ float4 row_score4(const float4 *lut, uint4 w) {
     return total;
 }
 
-template <int MT, int DS>
+template <int MT, int M, int DS>
 __global__ __launch_bounds__(kListThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_ivfpq_lists(ListArgs L) {
-    constexpr int M = 16, KS = 256, QB = kListQb, CH = kListChunkRows;
+    constexpr int KS = 256, QB = kListQb, CH = kListChunkRows;
     static_assert(kListThreads == KS && CH == 4 * 64 && QB == 4, "a thread per table entry; a row per lane");
     const ScanArgs &A = L.s;
-    __shared__ __attribute__((aligned(16))) ListLds S;
+    __shared__ __attribute__((aligned(16))) ListLds<M> S;
     static_assert(QB * 128 * sizeof(float) <= sizeof(S.cand), "residuals of dim <= 128 fit");
     float *s_r = reinterpret_cast<float *>(S.cand);  // residuals, before the scan
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -690,11 +715,12 @@ __global__ __launch_bounds__(kListThreads) __attribute__((amdgpu_waves_per_eu(2)
     constexpr bool hib = hib_metric(MT);
 
     // sub-centroid tid of every sub-space, DS floats each (thread-major layout)
-    float cbr[kLutRegs];
+    static_assert(M * DS <= kLutRegs, "the codebook column fits its registers");
+    float cbr[M * DS];
     {
         const float4 *src = reinterpret_cast<const float4 *>(A.cbt + (size_t)tid * kLutRegs);
 #pragma unroll
-        for (int v = 0; v < kLutRegs / 4; ++v) {
+        for (int v = 0; v < M * DS / 4; ++v) {
             const float4 f = src[v];
             cbr[4 * v] = f.x;
             cbr[4 * v + 1] = f.y;
@@ -735,14 +761,14 @@ __global__ __launch_bounds__(kListThreads) __attribute__((amdgpu_waves_per_eu(2)
         // chunk c's loads: this lane's code row (row 64 wave + lane), the ids of the rows the wave
         // offers (rows lane + 64 st; rows past the list's end repeat its last row, never used) and
         // the score word of the query's k-th best key as other pairs have left it so far
-        auto load_chunk = [&](int c, uint4 &w, uint32_t (&id)[4], uint32_t &th) {
+        auto load_chunk = [&](int c, CodeRow<M / 4> &w, uint32_t (&id)[4], uint32_t &th) {
             const uint32_t r = min((uint32_t)(c * CH + 64 * wave + lane), len - 1);
-            w = *reinterpret_cast<const uint4 *>(A.codes + (size_t)(beg + r) * 16);
+            w = load_code_row<M / 4>(A.codes + (size_t)(beg + r) * M);
 #pragma unroll
             for (int st = 0; st < 4; ++st) id[st] = A.ids[beg + min((uint32_t)(c * CH + 64 * st + lane), len - 1)];
             th = __hip_atomic_load(tau_hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         };
-        uint4 wa, wb;
+        CodeRow<M / 4> wa, wb;
         uint32_t ida[4], idb[4], tha, thb;
         // the first chunk's loads are in flight during the table build, except for cosine, whose
         // build needs their registers (three sums a step) to stay at two waves per SIMD
@@ -788,8 +814,8 @@ __global__ __launch_bounds__(kListThreads) __attribute__((amdgpu_waves_per_eu(2)
         lds_barrier();
         // chunk c: score this wave's rows for the four pairs, then (after the barrier) offer pair
         // `wave`'s 256 scores
-        auto do_chunk = [&](int c, const uint4 &w, const uint32_t (&id)[4], uint32_t ext_hi) {
-            const float4 t4 = row_score4(S.lut, w);
+        auto do_chunk = [&](int c, const CodeRow<M / 4> &w, const uint32_t (&id)[4], uint32_t ext_hi) {
+            const float4 t4 = row_score4<M / 4>(S.lut, w);
             float *sc = &S.score[c & 1][0][64 * wave + lane];
             sc[0 * CH] = t4.x;
             sc[1 * CH] = t4.y;
@@ -885,15 +911,26 @@ __global__ __launch_bounds__(256) void k_ivfpq_merge(ListArgs L, int P) {
     }
 }
 
+template <int MT, int M, int DS>
+void launch_lists_shape(const ListArgs &L, int cus, hipStream_t s) {
+    // persistent: as many workgroups as fit (each CU holds 163840 bytes of LDS, and two waves a SIMD of
+    // this kernel's registers)
+    const size_t per_cu = std::max<size_t>(1, std::min<size_t>(2, 163840 / (sizeof(ListLds<M>) + 256)));
+    const unsigned grid = (unsigned)((size_t)cus * per_cu);
+    scan_launch((k_ivfpq_lists<MT, M, DS>), dim3(grid), dim3(kListThreads), 0, s, L);
+}
+
+// The shapes list_path() admits: 16-byte rows of sub-vectors of 4 or 8 floats, 8-byte rows of 4, 8 or 16.
 template <int MT>
 void launch_lists_mt(const ListArgs &L, int ds, int cus, hipStream_t s) {
-    // persistent: as many workgroups as fit (each CU holds 163840 bytes of LDS)
-    const size_t per_cu = std::max<size_t>(1, 163840 / (sizeof(ListLds) + 256));
-    const unsigned grid = (unsigned)((size_t)cus * per_cu);
-    if (ds == 4)
-        scan_launch((k_ivfpq_lists<MT, 4>), dim3(grid), dim3(kListThreads), 0, s, L);
-    else
-        scan_launch((k_ivfpq_lists<MT, 8>), dim3(grid), dim3(kListThreads), 0, s, L);
+    if (L.s.m_sub == 16) {
+        if (ds == 4) launch_lists_shape<MT, 16, 4>(L, cus, s);
+        else launch_lists_shape<MT, 16, 8>(L, cus, s);
+    } else {
+        if (ds == 4) launch_lists_shape<MT, 8, 4>(L, cus, s);
+        else if (ds == 8) launch_lists_shape<MT, 8, 8>(L, cus, s);
+        else launch_lists_shape<MT, 8, 16>(L, cus, s);
+    }
 }
 
 template <bool HIB>
@@ -953,7 +990,7 @@ inline size_t scan_lds_bytes(size_t dim, size_t m_sub, size_t ks, int capw, int 
 void launch_ivfpq_scan_l2(const ScanArgs &A, int ds, int nv, int cus, size_t lds, hipStream_t s);
 void launch_ivfpq_scan_ip(const ScanArgs &A, int ds, int nv, int cus, size_t lds, hipStream_t s);
 void launch_ivfpq_scan_mem(const ScanArgs &A, int nv, int cus, size_t lds, hipStream_t s);
-// List-major scan and merge (16-byte code rows, 256 sub-centroids, ds 4 or 8, k <= kListMaxK,
+// List-major scan and merge (the shapes of launch_lists_mt, 256 sub-centroids, k <= kListMaxK,
 // nprobe * k <= kListMaxMerge); the plan (pairs, items, counters) is built by ivfpq_list_plan.
 void launch_ivfpq_lists_l2(const ListArgs &L, int ds, int cus, hipStream_t s);
 void launch_ivfpq_lists_ip(const ListArgs &L, int ds, int cus, hipStream_t s);
