@@ -14,7 +14,7 @@
 // padded to a multiple of 256 with NaN rows, so every score they produce is NaN and fails every
 // comparison; B's row count is padded to a multiple of 128.  The inner loop has no bounds checks.
 //
-// Two kernels share the epilogues:
+// Four kernels share the epilogues:
 //  * k_mfma_hs (dpad <= 128): a workgroup of 8 waves owns a work item of 128 columns whose
 //    128 x dpad tile stays resident in LDS; each wave streams its own rows of A straight from
 //    L2 into registers one step ahead, so waves need no barrier inside an item, and computes its
@@ -23,6 +23,7 @@
 //  * k_mfma_pnl (dpad a multiple of 128 above 128): the same per-wave register feed of A; the
 //    column tile passes through double-buffered LDS in K-panels of 128 floats, copied by
 //    global_load_lds one panel ahead, with one barrier per panel.
+//  * k_mfma_nt (searches at dpad 160 to 896): 32 columns resident in LDS, see below.
 //  * k_mfma_stream (other dpad > 128): a workgroup of 4 waves streams 128-row x 128-column
 //    stages of both operands through double-buffered LDS in K-chunks (32 flop per byte), two
 //    workgroups per CU.
