@@ -14,9 +14,9 @@
 //      kmeans.hip, summed with LDS integer atomics (exact in any order) and written per workgroup;
 //   3. k_pq_finalize -- the workgroups' sums added up, new = old + sum / count, the centroid's shift.
 // Bound: the vector ALUs in the assignment.  65,536 x 128 points, 8 sub-spaces of 256 centroids, 10
-// iterations, host data in, codebooks out: 21 ms by sub-space k-means, 3.3 here (1.7 of it the upload and allocations); an
-// assignment of all sub-spaces takes 129 us (94 at the rate of its subtracts and multiply-adds), the sums
-// 18, the new centroids 8. Encoding the same points: 524 us -> 134.
+// iterations, host data in, codebooks out: 21 ms by sub-space k-means, 3.3 here (1.7 of it the upload and
+// allocations); an assignment of all sub-spaces takes 129 us (94 at the rate of its subtracts and
+// multiply-adds), the sums 18, the new centroids 8.  Encoding the same points: 524 us -> 134.
 #include <algorithm>
 #include <cmath>
 #include <memory>
