@@ -1,4 +1,4 @@
-"""GPU tests of the list-major IVF-PQ scan (16-byte code rows, 256 sub-centroids, k <= 48).
+"""GPU tests of the list-major IVF-PQ scan (16- and 8-byte code rows, 256 sub-centroids, k <= 48).
 
 The list-major search groups the (query, probe) pairs by list and scores each list's codes once
 per batch of the queries probing it; the query-major kernel (forced with VHIP_IVFPQ_SCAN=query)
@@ -152,3 +152,22 @@ def test_eight_byte_rows_match_query_major(vh, metric, dim, k, nprobe, nq):
     ix = _index(vh, parts, dim, 8, 256, vh.DistanceMetric[metric])
     a, b = _both_paths(ix, rng.standard_normal((nq, dim)).astype(np.float32), k, nprobe)
     _assert_same(a, b)
+
+
+@pytest.mark.parametrize("m_sub,dim", [(16, 64), (16, 128), (8, 32), (8, 128)])
+@pytest.mark.parametrize("metric", ["L2Squared", "CosineSimilarity"])
+@pytest.mark.parametrize("empty", [(23,), (19, 20, 21, 22, 23), tuple(range(1, 24)), (0, 23)])
+def test_last_lists_empty(vh, m_sub, dim, metric, empty):
+    """No code row lies behind an empty last list, so its work items may load none: the last list
+    empty, the last five, all but the first (one row in all), the first and the last."""
+    rng = np.random.default_rng(dim + 100 * m_sub + len(empty))
+    nlist = 24
+    n = 1 if len(empty) == nlist - 1 else 3000
+    parts = _skewed_parts(rng, dim, nlist, n, empty=empty, m_sub=m_sub)
+    assert all(parts[2][c] == 0 for c in empty)
+    ix = _index(vh, parts, dim, m_sub, 256, vh.DistanceMetric[metric])
+    qs = rng.standard_normal((1100, dim)).astype(np.float32)
+    for nprobe in (1, 24):
+        a, b = _both_paths(ix, qs, 10, nprobe)
+        _assert_same(a, b)
+    assert np.all(a[2] == min(n, 10)), "every list was probed"

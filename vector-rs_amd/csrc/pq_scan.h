@@ -760,12 +760,16 @@ __global__ __launch_bounds__(kListThreads) __attribute__((amdgpu_waves_per_eu(2)
         const uint32_t *tau_hi = reinterpret_cast<const uint32_t *>(L.tau_q + qid) + 1;
         // chunk c's loads: this lane's code row (row 64 wave + lane), the ids of the rows the wave
         // offers (rows lane + 64 st; rows past the list's end repeat its last row, never used) and
-        // the score word of the query's k-th best key as other pairs have left it so far
+        // the score word of the query's k-th best key as other pairs have left it so far.  An empty
+        // list has no row to repeat and may be the last one, with no row of another list behind it:
+        // its first chunk's loads, which nothing uses, read the index's row 0 (an index without
+        // rows is not searched).
+        const uint32_t row0 = len ? beg : 0u, last = max(len, 1u) - 1u;
         auto load_chunk = [&](int c, CodeRow<M / 4> &w, uint32_t (&id)[4], uint32_t &th) {
-            const uint32_t r = min((uint32_t)(c * CH + 64 * wave + lane), len - 1);
-            w = load_code_row<M / 4>(A.codes + (size_t)(beg + r) * M);
+            const uint32_t r = min((uint32_t)(c * CH + 64 * wave + lane), last);
+            w = load_code_row<M / 4>(A.codes + (size_t)(row0 + r) * M);
 #pragma unroll
-            for (int st = 0; st < 4; ++st) id[st] = A.ids[beg + min((uint32_t)(c * CH + 64 * st + lane), len - 1)];
+            for (int st = 0; st < 4; ++st) id[st] = A.ids[row0 + min((uint32_t)(c * CH + 64 * st + lane), last)];
             th = __hip_atomic_load(tau_hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         };
         CodeRow<M / 4> wa, wb;
