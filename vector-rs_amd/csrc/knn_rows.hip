@@ -39,6 +39,13 @@ constexpr int kScanQueries = 16;   // queries of a tile
 constexpr int kScanFew = 4;        // in a round of few workgroups (its rows spread over more of them)
 constexpr long kScanFewWgs = 512;  // fewer workgroups of 16-query tiles than this (two a CU): 4-query tiles
 constexpr long kScanMaxWgs = 1L << 22;  // workgroups of a launch (a dispatch counts its threads in 32 bits)
+// Queries that an XCD's row groups take in turn before the next ones: half of its 4 MB L2, the row groups
+// in flight have the rest.  Whole searches, k = 10, without this limit -> 3, 2, 1 and 0.5 MB:
+//   L1      300,000 x 128, 10,000 queries (5.1 MB)   22.0 ms -> 15.5, 15.3, 15.4, 15.5
+//   L1      60,000 x 300,  4,000 queries (5.1 MB)     3.97   ->  3.19, 3.05, 3.08, 3.14;  1,000 queries 0.85 -> 0.84, 0.84, 0.88, 0.90
+//   L1      20,000 x 1,000, 4,000 queries (16 MB)     4.00   ->  3.89, 3.83, 3.81, 3.81
+//   Jaccard 300,000 x 128, 10,000 queries            42.7    -> 37.3, 37.2, 37.2, 37.2
+constexpr long kScanQueryBytes = 2L << 20;
 constexpr int kScanSlots = 16;     // LDS candidate slots per query and workgroup
 constexpr int kScanWg = 256;       // rows per workgroup: 4 waves of 64 rows, one a lane
 
@@ -53,17 +60,22 @@ struct RowScanArgs {
     uint32_t *cnt;        // FILTER: per-query candidate counters, cnt_stride words apart
     int cnt_stride, cap;
     long cand_row0;       // DENSE: row r goes to slot r - cand_row0
-    int n_groups, n_qtiles, spread;  // row groups, query tiles, and how workgroups map to them
+    int n_groups, n_qtiles, spread, chunk;  // row groups, query tiles, and how workgroups map to them
 };
 
 // (row group, query tile) of a workgroup.  spread: an XCD (workgroups b mod 8) takes every eighth row
-// group and runs all its query tiles one after another, so a group's rows are read into one L2 once.
+// group; it runs `chunk` query tiles (the last chunk what is left) of its first group one after another,
+// then of its next, and so through all its groups before the next chunk, so the group's rows and the
+// chunk's queries stay in its L2.
 __device__ __forceinline__ bool scan_tile(const RowScanArgs &a, int &group, int &qt) {
     const unsigned b = blockIdx.x;
     if (a.spread) {
-        const unsigned seq = b >> 3;
-        group = (int)(seq / (unsigned)a.n_qtiles * 8u + (b & 7u));
-        qt = (int)(seq % (unsigned)a.n_qtiles);
+        const unsigned seq = b >> 3, per_xcd = (unsigned)(a.n_groups + 7) / 8u;  // row groups of an XCD
+        const unsigned first = seq / (per_xcd * (unsigned)a.chunk) * (unsigned)a.chunk;
+        const unsigned tiles = min((unsigned)a.chunk, (unsigned)a.n_qtiles - first);
+        const unsigned at = seq - per_xcd * first;
+        group = (int)(at / tiles * 8u + (b & 7u));
+        qt = (int)(first + at % tiles);
         return group < a.n_groups;
     }
     group = (int)(b % (unsigned)a.n_groups);
@@ -325,15 +337,21 @@ __global__ __launch_bounds__(kScanWg) void k_ham_rows(RowScanArgs a) {
 template <class K>
 static void launch_rows(K kernel, RowScanArgs a, int nq_tile, long group_rows, hipStream_t s) {
     a.n_qtiles = ceil_div(a.nq, nq_tile);
+    a.chunk = (int)std::clamp(kScanQueryBytes / (4L * nq_tile * a.dpad), 1L, (long)a.n_qtiles);
     const long re = a.row_end;
     const long most = std::max(1L, kScanMaxWgs / a.n_qtiles / 8 * 8) * group_rows;  // rows of one launch
     for (long rb = a.row_begin; rb < re; rb += most) {
         a.row_begin = rb;
         a.row_end = std::min(re, rb + most);
         a.n_groups = (int)((a.row_end - rb + group_rows - 1) / group_rows);
-        // Eight or more groups an XCD balance; fewer spread over the whole chip in plain order.
-        a.spread = a.n_groups >= 64 && a.n_qtiles > 1;
-        const long wgs = (a.spread ? (a.n_groups + 7) / 8 * 8L : (long)a.n_groups) * a.n_qtiles;
+        // Spread where the XCDs' shares differ by little: eight or more groups an XCD, or idle places at
+        // most 8% of the groups.  Otherwise, in plain order, the whole chip shares them, and each XCD reads
+        // every group.  (From 64 groups on alone: L1 20,000 x 128, whose filter rounds have 24 and 47
+        // groups, 4,000 queries 682 us, with the second rule 575; spread over 16 places, the 12 groups of
+        // 5,000 x 128 229 -> 250.)
+        const long places = (a.n_groups + 7) / 8 * 8L;
+        a.spread = a.n_qtiles > 1 && (a.n_groups >= 64 || (places - a.n_groups) * 100 <= a.n_groups * 8L);
+        const long wgs = (a.spread ? places : (long)a.n_groups) * a.n_qtiles;
         scan_launch(kernel, dim3((unsigned)wgs), dim3(kScanWg), 0, s, a);
     }
 }
