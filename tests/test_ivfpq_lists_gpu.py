@@ -171,3 +171,17 @@ def test_last_lists_empty(vh, m_sub, dim, metric, empty):
         a, b = _both_paths(ix, qs, 10, nprobe)
         _assert_same(a, b)
     assert np.all(a[2] == min(n, 10)), "every list was probed"
+
+
+@pytest.mark.parametrize("nlist,n,k,nprobe,nq", [(64, 20_000, 10, 4, 1024), (64, 20_000, 10, 4, 1025), (64, 20_000, 10, 2, 1024),
+                                                 (16, 40_000, 10, 8, 1024), (1500, 30_000, 10, 2, 1499),
+                                                 (1500, 30_000, 10, 2, 1500), (2100, 30_000, 20, 3, 4199),
+                                                 (2100, 30_000, 20, 3, 4200), (64, 10_000, 48, 21, 4096),
+                                                 (64, 10_000, 48, 22, 4096)])
+def test_eight_byte_rows_around_the_choice_of_path(vh, nlist, n, k, nprobe, nq):
+    """Both sides of the batch sizes, list counts and k x nprobe at which 8-byte rows change paths."""
+    rng = np.random.default_rng(nlist + nq)
+    parts = _skewed_parts(rng, 64, nlist, n, m_sub=8)
+    ix = _index(vh, parts, 64, 8, 256, vh.DistanceMetric.L2Squared)
+    a, b = _both_paths(ix, rng.standard_normal((nq, 64)).astype(np.float32), k, nprobe)
+    _assert_same(a, b)

@@ -461,20 +461,42 @@ void ivfpq_list_plan(const uint32_t *probes, int nq, int nprobe, int nlist, cons
 
 // The list-major search applies to code rows of 16 or 8 bytes of 256 sub-centroids with the register-held
 // codebook (ds 4 or 8, with 8-byte rows also 16) and k <= kListMaxK; VHIP_IVFPQ_SCAN=query forces the
-// query-major kernel.  With 8-byte rows a table holds half as much, so the query-major kernel, one
-// workgroup a query and 512 resident, keeps up until they have run twice over (later for a larger k, whose
-// merge of nprobe k keys costs the list-major search more).  Whole searches, query-major / list-major us:
-//   400k x 128, nlist 512, nprobe 16, k = 10:  500 queries 162 / 216,  2,000 405 / 373,  8,000 1374 / 995
-//   400k x 32, the same:                       500 151 / 182,          2,000 395 / 310,  8,000 1374 / 820
-//   300k x 64, nlist 512, nprobe 4, k = 1:     500 107 / 134,          2,000 232 / 180,  8,000 734 / 352
-//   100k x 128, nlist 64, nprobe 8, k = 40:    500 156 / 243,          2,000 389 / 447,  8,000 1326 / 1204
+// query-major kernel.  16-byte rows always take it, 8-byte rows where lists8_pay().
+//
+// 8-byte rows.  A table holds half as much, so the query-major kernel, one workgroup a query and 512
+// resident, is ahead while they run at most twice over: the list-major search has about 70 us of fixed
+// cost (plan, merge, four tables an item however few pairs it has).  Whole searches of 21 shapes of
+// index from 20,000 to 2,000,000 rows in 32 to 8,192 lists, nprobe 1 to 64, query-major / list-major us:
+//   * up to 1,024 queries (two turns of the residents) it is behind, e.g. 400k x 128, nlist 1,024, nprobe 4,
+//     k = 10: 1,024 queries 158 / 194; from the third turn on ahead: 150k x 128, nlist 512, the same:
+//     1,300 queries 188 / 171.  At 1,024 queries it is ahead already where a query scans 16,384 codes or
+//     more (400k x 64, nlist 256, nprobe 64: 774 / 464) or probes one or two of few long lists (100k x 32,
+//     nlist 64, nprobe 1: 159 / 128);
+//   * it needs a query for every list, for every two where lists have 256 rows or more, to fill its
+//     items: 400k x 128, nlist 4,096, nprobe 4, k = 10: 2,000 queries 220 / 288, 4,096 342 / 369, 10,000
+//     779 / 662; 800k x 128, nlist 2,048: 1,300 queries, nprobe 6: 227 / 215;
+//   * for k > 16 its merge of nprobe k keys a query costs more: 100k x 128, nlist 64, nprobe 8, k = 48:
+//     2,000 queries 423 / 512, 10,000 1767 / 1732; most where lists are short (400k x 128, nlist 4,096,
+//     nprobe 64: 10,000 queries 2849 / 3305).
+// Of 2,242 measured searches with 1,024 queries or more the rule takes list-major where it is more than 3%
+// slower 16 times, by 8% at most; from 1,024 queries on (4,096 for k > 16) alone it was 331 times, by up to 61%.
 constexpr size_t kListMinQueries8 = 1024, kListMinQueries8LargeK = 4096, kListSmallK8 = 16;
+constexpr size_t kListLongRows = 256, kListManyCodes = 16384;
+static bool lists8_pay(size_t n, size_t nlist, size_t nq, size_t k, size_t np) {
+    const size_t rows = n / nlist;  // of a list, on average
+    const bool long_lists = rows >= kListLongRows;
+    const size_t fill = long_lists ? nlist / 2 : nlist;
+    if (k > kListSmallK8)
+        return nq >= std::max(kListMinQueries8LargeK, 2 * fill) && (long_lists || np * k <= 1024);
+    const bool early = np * rows >= kListManyCodes || (np <= 2 && nlist <= 256 && long_lists);
+    return nq >= std::max(kListMinQueries8 + (early ? 0 : 1), fill);
+}
 static bool list_path(const vhip_ivfpq *X, size_t nq, size_t k, size_t np) {
     if (const char *e = std::getenv("VHIP_IVFPQ_SCAN"))
         if (std::strcmp(e, "query") == 0) return false;
     const bool shape16 = X->m_sub == 16 && (X->ds == 4 || X->ds == 8);
     const bool shape8 = X->m_sub == 8 && (X->ds == 4 || X->ds == 8 || X->ds == 16) &&
-                        nq >= (k <= kListSmallK8 ? kListMinQueries8 : kListMinQueries8LargeK);
+                        lists8_pay(X->n, X->nlist, nq, k, np);
     return X->reg && X->ks == 256 && (shape16 || shape8) && k >= 1 && k <= (size_t)kListMaxK &&
            np * k <= (size_t)kListMaxMerge && sizeof(ListLds<16>) <= X->lds_limit;
 }

@@ -68,13 +68,13 @@ constexpr int ring_chunk_bytes(int nv) { return nv * 1024 + 256; }
 constexpr int ring_bytes(int nv) { return kScanWaves * ring_chunks(nv) * ring_chunk_bytes(nv); }
 
 // ---- list-major scan --------------------------------------------------------------------------
-// For 16-byte code rows (16 sub-spaces of 256 sub-centroids) and k <= kListMaxK the search runs
+// For code rows of 16 bytes, or of 8 where pq.hip's list_path says so, and k <= kListMaxK the search runs
 // list-major: the (query, probe) pairs are grouped by list, and a work item is one list with up to
 // kListQb of the queries probing it.  The item's kListQb ADC tables are built in LDS side by side:
 // entry (m, e) of the four tables is one float4 (thread j computes sub-centroid j's entries from its
 // register-held codebook), so one 16-byte LDS read per code byte serves the item's four pairs.  The
 // list then streams once: wave w scores rows 64 w .. 64 w + 63 of each 256-row chunk, one row a
-// lane (its 16 code bytes loaded straight into registers, one chunk ahead), against the four
+// lane (its code bytes loaded straight into registers, one chunk ahead), against the four
 // tables with the summation order of compute_distance_with_lut (pq.rs:270-293), and leaves the
 // four scores in LDS; after one barrier per chunk, wave q filters and offers the chunk's 256
 // scores of pair q, keeping its k best.  A list's codes are therefore read once per kListQb probing
@@ -917,8 +917,9 @@ __global__ __launch_bounds__(256) void k_ivfpq_merge(ListArgs L, int P) {
 
 template <int MT, int M, int DS>
 void launch_lists_shape(const ListArgs &L, int cus, hipStream_t s) {
-    // persistent: as many workgroups as fit (each CU holds 163840 bytes of LDS, and two waves a SIMD of
-    // this kernel's registers)
+    // persistent: as many workgroups as fit a CU's 163840 bytes of LDS, two at most: two waves a SIMD of the
+    // registers of <., 16, 8> and <., 8, 16> (the narrower shapes' 126 to 166 registers would hold a third
+    // workgroup, which is not used)
     const size_t per_cu = std::max<size_t>(1, std::min<size_t>(2, 163840 / (sizeof(ListLds<M>) + 256)));
     const unsigned grid = (unsigned)((size_t)cus * per_cu);
     scan_launch((k_ivfpq_lists<MT, M, DS>), dim3(grid), dim3(kListThreads), 0, s, L);
