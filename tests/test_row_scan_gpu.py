@@ -81,6 +81,22 @@ def test_hamming_small_batches(vh, words, n, k):
         np.testing.assert_array_equal(d2[:, :kk], dist[:nq, :kk])
 
 
+@pytest.mark.parametrize("words,n,nq,k", [(2, 30_001, 7168, 1), (8, 30_001, 7169, 1), (32, 30_001, 7169, 40),
+                                          (8, 40_001, 5120, 1), (8, 40_001, 5121, 1), (2, 40_001, 5121, 70),
+                                          (32, 40_001, 2047, 1), (16, 40_001, 2048, 10), (8, 40_001, 14_337, 1)])
+def test_hamming_large_batches(vh, monkeypatch, words, n, nq, k):
+    """Both sides of the batch sizes from which the fp4 scan's first round has 1,024 or 512 rows, and k whose
+    20 k rows are more than that; the popcount batch kernel is the reference."""
+    rng = np.random.default_rng(words + nq)
+    codes = rng.integers(0, 1 << 32, (n, words), dtype=np.uint64).astype(np.uint32)
+    q = rng.integers(0, 1 << 32, (nq, words), dtype=np.uint64).astype(np.uint32)
+    ids, dist, _ = vh.HammingKnnEngine(codes).search_batch_arrays(q, k)
+    monkeypatch.setenv("VHIP_HAMMING_KERNEL", "popcount")
+    i2, d2, _ = vh.HammingKnnEngine(codes).search_batch_arrays(q, k)
+    np.testing.assert_array_equal(ids, i2)
+    np.testing.assert_array_equal(dist, d2)
+
+
 @pytest.mark.parametrize("words", [2, 8, 32])
 @pytest.mark.parametrize("nq", [17, 128, 129, 256])
 def test_hamming_mid_batches(vh, monkeypatch, words, nq):

@@ -102,8 +102,9 @@ struct vhip_knn {
 namespace vh {
 
 // Search rounds.  Round 0 scores rows [0, b0) with b0 about 20 k, the first 256-row multiple
-// at or above it and at least kFirstRows (all rows when the base has at most max(2048, 32 k)), densely
-// (every score written, no atomics); the popcount batch kernel alone filters it with tau = +inf.
+// at or above it and at least kFirstRows (fewer for large fp4 Hamming batches; all rows when the
+// base has at most max(2048, 32 k)), densely (every score written, no atomics); the popcount batch
+// kernel alone filters it with tau = +inf.
 // Every later round covers about 4 times the rows seen so far (the growth factor, see
 // kRoundGrowth) and keeps only rows scoring <= tau, the k-th best so far.  Because the base rows
 // are in a pseudo-random order, round i passes about k * (rows_i / seen_i) ~ 3 k candidates per
@@ -125,28 +126,49 @@ struct Round {
 // (2 slower).
 constexpr int kRoundGrowth = 4;
 
-// Small batches (`small`: at most kSmallCols queries on the GEMM metrics) pay mostly for launches
-// and merges, not for scanned pairs: their first, dense round covers kSmallDenseRows rows (all of a
-// base of up to twice that), and the rest follows in one filter round when its expected passes per
-// query, k (n - seen) / seen, stay within a quarter of the candidate capacity, else in rounds growing
-// 16 times.  (1M rows at k = 10: 8,192 rows, then the other 991,808 with about 1,200 passes; at
-// k = 100 three rounds.)  A larger first round costs more in its merge (32,768 rows: 27 us against
-// about 12) than the fewer passes save.
+// Small batches (`small`, see small_plan: small_batch() on the GEMM metrics, up to kValuSmallQueries on the
+// vector-ALU ones, up to kHamSmallRounds on packed codes) pay mostly for launches and merges, not for
+// scanned pairs: their first, dense round covers kSmallDenseRows rows (all of a base of up to twice
+// that), and the rest follows in one filter round when its expected passes per query, k (n - seen) /
+// seen, stay within a quarter of the candidate capacity, else in rounds growing 16 times.  (1M rows at
+// k = 10: 8,192 rows, then the other 991,808 with about 1,200 passes; at k = 100 three rounds.)  A larger
+// first round costs more in its merge (32,768 rows: 27 us against about 12) than the fewer passes save.
 constexpr size_t kSmallDenseRows = 8192;
 // A dense first round has at least this many rows: a small round costs about as much as its launch and
 // merge, whatever its rows, and 2,048 candidates a query is the lists' least capacity anyway.  Against a
 // start of 256 rows (512 at k = 20), whole searches: L1 500k x 128, 4,096 queries 10528 -> 10163 us; dot
 // 200,003 x 300, k = 20, 129 queries 346 -> 309, 1,000 1171 -> 1136; cosine 20,000 x 64, 1,000 queries
 // 170 -> 128, 8,000 486 -> 433; squared L2 1M x 128, 8,000 queries 14901 -> 14835; fp4 Hamming 4M x 256
-// bits, 512 queries 426 -> 397, 10,000 3793 -> 3776 (100k x 256: 10,000 queries 516 -> 525).
+// bits, 512 queries 426 -> 397.
 constexpr size_t kFirstRows = 2048;
+// fp4 Hamming scores a row so cheaply that for large batches writing and merging 2,048 scores of each query
+// (117 MB at 7,168) costs as much as the rounds it saves.  Against a start of 256 rows, rounds of four
+// times the rows seen give: 2,048 rows one round fewer or two, by the base's size; 512 none or one; 1,024
+// always one.  Where 2,048 saves two it pays up to kHamFirstQueries queries, and 512 rows above; where it
+// saves one, up to kHamFirstQueriesWide (kHamFirstQueriesTile where ham_wide is off), 1,024 rows above
+// and 512 for the largest batches.  Whole searches, k = 1, starts of 256 / 512 / 1,024 / 2,048 rows, us:
+//   saves two:  100k x 256 bits: 7,000 queries 293 / 282 / 287 / 273, 12,000 399 / 371 / 392 / 435, 16,384
+//               460 / 433 / 507 / 552
+//   saves one:  200k x 256 bits: 5,000 queries 306 / 297 / 300 / 278, 10,000 429 / 421 / 412 / 480;
+//               800k x 512 bits: 1,000 queries 283 / 292 / 278 / 283, 5,000 913 / 931 / 949 / 995
+constexpr size_t kHamFirstQueries = 7168, kHamFirstQueriesWide = 5120, kHamFirstQueriesTile = 2047;
+static size_t ham_first_rows(size_t n, size_t nq, bool wide) {
+    size_t end = kFirstRows;  // of the rounds of a 2,048-row start: the first at or past n
+    while (end < n) end *= kRoundGrowth;
+    const bool saves_two = n > end / 2;  // the 256-row start's last rounds end at end / 2 and at 2 end
+    if (nq <= (saves_two ? kHamFirstQueries : (wide ? kHamFirstQueriesWide : kHamFirstQueriesTile))) return kFirstRows;
+    return saves_two || nq > 2 * kHamFirstQueries ? kFirstRows / 4 : kFirstRows / 2;
+}
+// A filtered first round (the popcount batch kernel's).
+constexpr size_t kFilterFirstRows = 256;
 
-static std::vector<Round> plan_rounds(size_t n, size_t k, bool dense0, int dpad, int growth,
+// first: the least rows of the first round; dense0: that round writes every score.
+static std::vector<Round> plan_rounds(size_t n, size_t k, size_t first, bool dense0, int dpad, int growth,
                                       bool small = false) {
     std::vector<Round> r;
     if (n == 0) return r;
     const size_t kk = std::max<size_t>(k, 1);
-    size_t b0 = std::min(n, round_up(std::max<size_t>(dense0 ? kFirstRows : 256, 20 * kk), kRowAlign));
+    size_t b0 = std::min(n, round_up(std::max<size_t>(first, 20 * kk), kRowAlign));
     // A base within the candidate capacity's floor (round_cap) is scored in one dense round: its
     // later rounds would cost more launches than rows (the IVF coarse probe: 1,024 centroids).
     if (n <= std::max<size_t>(2048, 32 * kk)) b0 = n;
@@ -191,7 +213,7 @@ static long balanced_item(long cap_item, long rows, int n_ctiles, int wgs, long 
 
 static int round_cap(size_t n, size_t k, int dpad, bool small) {
     size_t cap = std::max<size_t>(2048, 32 * std::max<size_t>(k, 1));
-    for (const Round &r : plan_rounds(n, k, true, dpad, kRoundGrowth, small))
+    for (const Round &r : plan_rounds(n, k, kFirstRows, true, dpad, kRoundGrowth, small))
         if (r.rb == 0) cap = std::max(cap, (size_t)(r.re - r.rb));
     return (int)round_up(cap, kRowAlign);
 }
@@ -375,9 +397,11 @@ static uint32_t first_count(const std::vector<Round> &rounds) {
     return !rounds.empty() && rounds[0].dense ? (uint32_t)(rounds[0].re - rounds[0].rb) : 0u;
 }
 // The rounds of a run.  The first is dense on every path but the popcount batch kernel's.
-static std::vector<Round> run_plan(const vhip_knn *E, int k, bool small, long max_round_rows) {
+static std::vector<Round> run_plan(const vhip_knn *E, size_t nq, int k, bool small, long max_round_rows) {
     const bool dense0 = E->metric != HAMMING_PACKED || E->ham8 || small;
-    return split_rounds(plan_rounds(E->n, (size_t)k, dense0, (int)E->dpad, kRoundGrowth, small), max_round_rows);
+    const size_t first = !dense0 ? kFilterFirstRows : (E->ham8 ? ham_first_rows(E->n, nq, E->ham_wide) : kFirstRows);
+    return split_rounds(plan_rounds(E->n, (size_t)k, first, dense0, (int)E->dpad, kRoundGrowth, small),
+                        max_round_rows);
 }
 
 // Runs all rounds for nq prepared queries; results stay in B.topk (row stride kc) / B.have.
@@ -390,7 +414,7 @@ static int run_rounds(vhip_knn *E, const QueryRows &Q, int nq, int k, int kc, in
                       const RunBufs &B, long max_round_rows, bool timed, bool reset_done = false) {
     hipStream_t s = E->stream;
     const bool gemm = is_gemm_metric(E->metric) && !direct;
-    const std::vector<Round> rounds = run_plan(E, k, small, max_round_rows);
+    const std::vector<Round> rounds = run_plan(E, (size_t)nq, k, small, max_round_rows);
     if (!reset_done)
         launch_topk_init(nq, B.tau, B.have, B.cnt, B.flags, B.mflag, B.nflag, first_count(rounds), B.spad, s);
     const bool small_scan = small_scan_run(E, (size_t)nq, direct);
@@ -482,9 +506,10 @@ static int run_rounds(vhip_knn *E, const QueryRows &Q, int nq, int k, int kc, in
 // plan.
 static int full_cap(const vhip_knn *E, size_t k) {
     long big = k;
-    for (int v = 0; v < 4; ++v)
-        for (const Round &rd : plan_rounds(E->n, k, (v & 1) != 0, (int)E->dpad, kRoundGrowth, (v & 2) != 0))
-            big = std::max(big, rd.re - rd.rb);
+    for (size_t first : {kFilterFirstRows, kFirstRows / 4, kFirstRows / 2, kFirstRows})
+        for (bool small : {false, true})
+            for (const Round &rd : plan_rounds(E->n, k, first, true, (int)E->dpad, kRoundGrowth, small))
+                big = std::max(big, rd.re - rd.rb);
     return (int)round_up((size_t)big, kRowAlign);
 }
 
@@ -893,7 +918,7 @@ static int engine_search_locked(vhip_knn *E, const void *d_queries, size_t nq, s
         }
         // the batch's run starts here too (search_prepared's first run_rounds skips its reset)
         rp.init = {bm.B.tau, bm.B.have, bm.B.cnt, bm.B.flags, bm.B.mflag, bm.B.nflag, bm.B.spad,
-                   first_count(run_plan(E, kk, small, 0))};
+                   first_count(run_plan(E, (size_t)m, kk, small, 0))};
         launch_rows_prep(rp, E->stream);
         VH_HIP(hipGetLastError());
         const QueryRows Q{bm.qpad, bm.qnorm, bm.qerr, E->shifted ? bm.qraw : bm.qpad};
