@@ -58,6 +58,24 @@ def test_sub_spaces_stop_by_themselves(vh):
     np.testing.assert_allclose(got[1], c, rtol=1e-6)
 
 
+def test_threads_train_with_different_cluster_counts(vh):
+    """Trainings that need 39, 65 and 98 KB of LDS a workgroup, at the same time."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    rng = np.random.default_rng(9)
+    x = rng.integers(-60, 60, (4000, 64)).astype(np.float32)
+    jobs = [100, 256, 170, 256, 100, 256, 170, 256]
+
+    def run(ks):
+        return vh.ProductQuantizer.train(x, 64, 2, ks, 6, -1.0, seed=3).codebooks
+
+    alone = {ks: run(ks) for ks in set(jobs)}
+    with ThreadPoolExecutor(max_workers=4) as ex:
+        for _ in range(4):
+            for ks, got in zip(jobs, ex.map(run, jobs)):
+                np.testing.assert_array_equal(got, alone[ks])
+
+
 def test_infinite_values_are_refused(vh):
     x = np.zeros((300, 8), np.float32)
     x[7, 5] = np.inf

@@ -266,6 +266,11 @@ __global__ __launch_bounds__(kPqThreads) void k_pq_finalize(float *__restrict__ 
     if (live && d == 0) shifts[m * k + c] = sh;
 }
 
+// Dynamic LDS of k_pq_sums<dsp> for k clusters: sums, scales and centroids.
+constexpr size_t pq_sums_lds(size_t dsp, size_t k) { return k * dsp * 8 + k * 8 + k * dsp * 4; }
+
+static_assert(pq_sums_lds(16, kPqMaxK) <= 65536 && pq_sums_lds(32, kPqMaxK) <= 163840, "LDS of a workgroup");
+
 int padded_ds(size_t ds) { return ds <= 4 ? 4 : (ds <= 8 ? 8 : (ds <= 16 ? 16 : 32)); }
 
 // Codebooks [m_sub][rows of ds floats, `have` per sub-space at stride `ks`] into [m_sub][have][DSP].
@@ -400,7 +405,12 @@ int pq_train_batched(int ordinal, const float *data, size_t n, size_t dim, size_
     VH_HIP(hipMemcpyAsync(&nonfinite, bad, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     VH_HIP(hipStreamSynchronize(s));
     if (nonfinite) return set_error(VHIP_ERR_INVALID_CONFIG, "data contains non-finite values");
-    const size_t lds = kd * 8 + ek * 8 + kd * 4;
+    const size_t lds = pq_sums_lds(dsp, ek);
+    // Only the widest kernel can need more than 64 KB.  Its limit is shared by every thread that trains, so
+    // it is set to the most that any cluster count needs, not to this call's.
+    if (dsp == 32)
+        VH_HIP(hipFuncSetAttribute((const void *)k_pq_sums<32>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)pq_sums_lds(32, kPqMaxK)));
     std::vector<uint32_t> on(m_sub, 1u);
     std::vector<float> sh(m_sub * ek);
     for (size_t it = 0; it < max_iters; ++it) {
@@ -408,8 +418,6 @@ int pq_train_batched(int ordinal, const float *data, size_t n, size_t dim, size_
     do {                                                                                                               \
         launch_assign<L2, DSP, true>(xs, (long)n, DSP, (long)n * DSP, DSP, 1, cent, k,         \
                                      (int)m_sub, assign, 1, (long)n, count, devmax, active, s);          \
-        if (lds > 65536) VH_HIP(hipFuncSetAttribute((const void *)k_pq_sums<DSP>,                                      \
-                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));            \
         hipLaunchKernelGGL(k_pq_sums<DSP>, dim3((unsigned)parts, (unsigned)m_sub), dim3(kPqThreads), lds, s,           \
                            xs, (long)n, (long)per, cent, k, assign, count,       \
                            devmax, part, active);                                             \
