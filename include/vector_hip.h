@@ -323,7 +323,10 @@ int vhip_ivfpq_config_validate(const vhip_ivfpq_config *cfg, size_t dim);
  * M x Ks x (dim / M) floats, zero rows past min(Ks, n) (pq.rs:84-88).  Initial sub-centroids
  * are a seeded sample without replacement (KMeans::init_centroids_random, ivf/kmeans.rs:359-371,
  * draws from an unseeded thread_rng) or, with init_codebooks != NULL, the given
- * min(Ks, n) x ds rows of each sub-space (at stride Ks rows). */
+ * min(Ks, n) x ds rows of each sub-space (at stride Ks rows).  Under squared L2 with sub-vectors of at
+ * most 32 floats the sub-spaces are trained together, in groups where they would take more than half
+ * of the free device memory; the environment variable VHIP_PQ_TRAIN_BYTES sets another limit.  The
+ * codebooks do not depend on the groups. */
 int vhip_pq_train(int ordinal, const float *data, size_t n, size_t dim, size_t num_subvectors, size_t sub_clusters,
                   size_t max_iters, float tol, int metric, const float *init_codebooks, uint64_t seed,
                   float *out_codebooks);

@@ -76,6 +76,57 @@ def test_threads_train_with_different_cluster_counts(vh):
                 np.testing.assert_array_equal(got, alone[ks])
 
 
+# one sub-space at a time and several uploads (limit 1), groups of like and of unlike size, the limit just
+# below what all sub-spaces take
+@pytest.mark.parametrize("n,ds,m,ks,limit", [(70_000, 16, 8, 256, 1), (70_000, 16, 8, 256, 30 << 20),
+                                             (20_000, 5, 7, 100, 3 << 20), (300, 32, 3, 256, 1), (5000, 1, 64, 16, 2 << 20)])
+@pytest.mark.parametrize("tol", [-1.0, 1e-3])
+def test_groups_of_sub_spaces(vh, monkeypatch, n, ds, m, ks, limit, tol):
+    """Where device memory is short the sub-spaces are trained in groups: the same codebooks, bit for bit."""
+    rng = np.random.default_rng(n + m)
+    x = rng.standard_normal((n, m * ds)).astype(np.float32)
+    whole = vh.ProductQuantizer.train(x, m * ds, m, ks, 4, tol, seed=5).codebooks
+    monkeypatch.setenv("VHIP_PQ_TRAIN_BYTES", str(limit))
+    np.testing.assert_array_equal(vh.ProductQuantizer.train(x, m * ds, m, ks, 4, tol, seed=5).codebooks, whole)
+    x[n // 2, m * ds - 1] = np.inf  # in the last group
+    with pytest.raises(vh.InvalidConfig):
+        vh.ProductQuantizer.train(x, m * ds, m, ks, 4, tol, seed=5)
+
+
+def test_training_stays_within_its_memory(vh, monkeypatch):
+    """32 sub-spaces of one float, padded to four: 690 MB all at once, 17 MB a sub-space and upload."""
+    import ctypes
+    import threading
+
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free():
+        f, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(total)) == 0
+        return f.value
+
+    rng = np.random.default_rng(1)
+    x = rng.standard_normal((1_000_000, 32)).astype(np.float32)
+    vh.ProductQuantizer.train(x[:1000], 32, 32, 16, 1, -1.0)
+    monkeypatch.setenv("VHIP_PQ_TRAIN_BYTES", str(64 << 20))
+    before, least, done = free(), [1 << 62], threading.Event()
+
+    def watch():
+        while not done.is_set():
+            least[0] = min(least[0], free())
+
+    t = threading.Thread(target=watch)
+    t.start()
+    try:
+        vh.ProductQuantizer.train(x, 32, 32, 16, 2, -1.0)
+    finally:
+        done.set()
+        t.join()
+    used = before - least[0]
+    print(f"  training took {used >> 20} MB of device memory at most", flush=True)
+    assert 16 << 20 <= used < 150 << 20
+
+
 def test_infinite_values_are_refused(vh):
     x = np.zeros((300, 8), np.float32)
     x[7, 5] = np.inf

@@ -19,6 +19,7 @@
 // multiply-adds), the sums 18, the new centroids 8.  Encoding the same points: 524 us -> 134.
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <memory>
 #include <vector>
 
@@ -142,12 +143,14 @@ __global__ __launch_bounds__(kPqThreads) void k_pq_assign(const float *__restric
     }
 }
 
-// Rows [n][dim] of points into sub-space-major rows [m][n][DSP], zero past ds; bad is set when some
-// value is infinite (what the general engine's check rejects).
+// Rows i0 .. i0 + rows of the n points, [rows][dim] at x, into sub-space-major rows [m][n][DSP] of the
+// sub-spaces m0 .. m0 + m_sub, zero past ds; bad is set when some value is infinite (what the general
+// engine's check rejects).
 template <int DSP>
-__global__ __launch_bounds__(256) void k_pq_split(const float *__restrict__ x, long n, int dim, int ds, int m_sub,
-                                                  float *__restrict__ out, uint32_t *__restrict__ bad) {
-    const long total = n * m_sub * DSP;
+__global__ __launch_bounds__(256) void k_pq_split(const float *__restrict__ x, long rows, long i0, long n, int dim,
+                                                  int ds, int m0, int m_sub, float *__restrict__ out,
+                                                  uint32_t *__restrict__ bad) {
+    const long total = rows * m_sub * DSP;
     for (long t = blockIdx.x * 256L + threadIdx.x; t < total; t += gridDim.x * 256L) {
         // consecutive threads write a row's DSP values, then the next sub-space of the same point, so that
         // a point's row is read once
@@ -155,9 +158,9 @@ __global__ __launch_bounds__(256) void k_pq_split(const float *__restrict__ x, l
         const long r = t / DSP;
         const int m = (int)(r % m_sub);
         const long i = r / m_sub;
-        const float v = d < ds ? x[i * dim + (long)m * ds + d] : 0.0f;
+        const float v = d < ds ? x[i * dim + (long)(m0 + m) * ds + d] : 0.0f;
         if (fabsf(v) == INFINITY) *bad = 1;
-        out[((long)m * n + i) * DSP + d] = v;
+        out[((long)m * n + i0 + i) * DSP + d] = v;
     }
 }
 
@@ -334,25 +337,79 @@ int pq_encode_narrow(const float *d_x, size_t n, size_t dim, size_t m_sub, size_
     return VHIP_OK;
 }
 
+namespace {
+
+// Device memory of `g` sub-spaces trained at once, uploaded `slab` rows at a time, in one allocation (freeing
+// a large buffer takes about 0.24 ms): byte offsets of the uploaded rows, the points by sub-space, the partial
+// sums, centroids, shifts, counters (counts, deviations, active flags, bad) and assignments.
+struct PqGroupMem {
+    size_t raw, xs, part, cent, shift, state, assign, total = 0;
+    PqGroupMem(size_t n, size_t dim, size_t slab, size_t g, size_t ek, size_t dsp, size_t parts) {
+        auto take = [&](size_t bytes) {
+            const size_t o = total;
+            total += round_up(bytes, 256);
+            return o;
+        };
+        raw = take(slab * dim * sizeof(float));
+        xs = take(n * g * dsp * sizeof(float));
+        part = take(parts * g * ek * dsp * sizeof(unsigned long long));
+        cent = take(g * ek * dsp * sizeof(float));
+        shift = take(g * ek * sizeof(float));
+        state = take((2 * g * ek + g + 1) * sizeof(uint32_t));
+        assign = take(n * g);
+    }
+};
+
+// Points of a workgroup of the sums of g sub-spaces: about two workgroups a CU in all, at least 256 points.
+size_t pq_sum_points(int ordinal, size_t n, size_t g) {
+    const size_t want = std::max<size_t>(1, (size_t)device_grid_cap(ordinal) / g);
+    return std::max<size_t>(256, (n + want - 1) / want);
+}
+
+constexpr size_t kPqSlabBytes = (size_t)1 << 30;  // of an upload
+constexpr size_t kPqMinSlabBytes = (size_t)16 << 20;
+constexpr size_t kPqAskBytes = (size_t)1 << 30;   // a training set that takes less does not ask what is free
+constexpr size_t kPqMaxGroup = 65535;             // sub-spaces are a grid dimension
+
+// Device memory that training may take: half of what is free (the rest stays for the program's other
+// objects), or VHIP_PQ_TRAIN_BYTES.
+size_t pq_train_limit(size_t bytes) {
+    if (const char *e = std::getenv("VHIP_PQ_TRAIN_BYTES")) return (size_t)std::strtoull(e, nullptr, 10);
+    if (bytes <= kPqAskBytes) return bytes;
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
+        (void)hipGetLastError();
+        return bytes;
+    }
+    return free_b / 2;
+}
+
+}  // namespace
+
 // ProductQuantizer::train under squared L2 for sub-vectors of at most 32 dimensions: the same codebooks as
-// one vhip_kmeans_fit per sub-space (seed + 1 + m, shuffled start).
+// one vhip_kmeans_fit per sub-space (seed + 1 + m, shuffled start).  All sub-spaces at once where they fit
+// the device memory (about 4 (dim + 1) bytes a point beside an upload of at most 1 GiB, more where ds is
+// padded), else as many at a time as do, each group uploading the rows again; one at a time takes less
+// than the general engine does for it.
 int pq_train_batched(int ordinal, const float *data, size_t n, size_t dim, size_t m_sub, size_t ks, size_t max_iters,
                      float tol, const float *init_codebooks, uint64_t seed, float *out_codebooks) {
     if (n > 0x7fffffffull) return set_error(VHIP_ERR_INVALID_CONFIG, "k-means supports n < 2^31 points");
     const size_t ds = dim / m_sub, ek = std::min(ks, n);
     const int dsp = padded_ds(ds), k = (int)ek;
+    const size_t kd = ek * dsp;
     VH_CHECK(open_device(ordinal));
     hipStream_t s;
     VH_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     DevBuf mem;
     PinnedStager st;
+    std::vector<float> start, sh, fin;
+    std::vector<uint32_t> on;
     // declared after the buffers: the stream is drained and destroyed before they are released
     std::unique_ptr<ihipStream_t, void (*)(hipStream_t)> hold(s, [](hipStream_t q) {
         (void)hipStreamSynchronize(q);
         (void)hipStreamDestroy(q);
     });
     st.dev = ordinal;
-    std::vector<float> start;
     if (init_codebooks) {
         start = pad_codebooks(init_codebooks, m_sub, ks, ek, ds, dsp);
     } else {
@@ -365,97 +422,108 @@ int pq_train_batched(int ordinal, const float *data, size_t n, size_t dim, size_
             }
         }
     }
-    // workgroups of the sums: about two a CU over all sub-spaces, at least 256 points each
-    const size_t want = std::max<size_t>(1, (size_t)device_grid_cap(ordinal) / m_sub);
-    const size_t per = std::max<size_t>(256, (n + want - 1) / want);
-    const int parts = (int)((n + per - 1) / per);
-    const size_t kd = ek * dsp, words = 2 * m_sub * ek + m_sub + 1;  // counts, deviations, active flags, bad
-    // one allocation for all of it (freeing a large buffer takes about 0.24 ms): the upload, the points by
-    // sub-space, partial sums, centroids, shifts, counters and assignments
-    size_t off = 0;
-    auto take = [&](size_t bytes) {
-        const size_t o = off;
-        off += round_up(bytes, 256);
-        return o;
+    // sub-spaces at a time and rows an upload: the most that the limit allows and the allocation gives
+    size_t slab = std::min(n, std::max<size_t>(1, kPqSlabBytes / (dim * sizeof(float))));
+    const size_t slab_min = std::min(n, std::max<size_t>(1, kPqMinSlabBytes / (dim * sizeof(float))));
+    size_t group = std::min(m_sub, kPqMaxGroup);
+    auto layout = [&](size_t g) {
+        const size_t per = pq_sum_points(ordinal, n, g);
+        return PqGroupMem(n, dim, slab, g, ek, dsp, (n + per - 1) / per);
     };
-    const size_t o_raw = take(n * dim * sizeof(float)), o_xs = take(n * m_sub * dsp * sizeof(float)),
-                 o_part = take((size_t)parts * m_sub * kd * sizeof(unsigned long long)),
-                 o_cent = take(m_sub * kd * sizeof(float)), o_shift = take(m_sub * ek * sizeof(float)),
-                 o_state = take(words * sizeof(uint32_t)), o_assign = take(n * m_sub);
-    VH_CHECK(mem.ensure(ordinal, off));
-    char *const m0 = mem.as<char>();
-    float *raw = (float *)(m0 + o_raw), *xs = (float *)(m0 + o_xs), *cent = (float *)(m0 + o_cent),
-          *shifts = (float *)(m0 + o_shift);
-    unsigned long long *part = (unsigned long long *)(m0 + o_part);
-    uint8_t *assign = (uint8_t *)(m0 + o_assign);
-    uint32_t *count = (uint32_t *)(m0 + o_state), *devmax = count + m_sub * ek, *active = devmax + m_sub * ek,
-             *bad = active + m_sub;
-    launch_fill_u32(count, 2 * m_sub * ek, 0u, s);
-    launch_fill_u32(active, m_sub, 1u, s);
-    launch_fill_u32(bad, 1, 0u, s);
-    VH_CHECK(st.h2d_once(raw, data, n * dim * sizeof(float), s));
-    VH_HIP(hipMemcpyAsync(cent, start.data(), start.size() * sizeof(float), hipMemcpyHostToDevice, s));
-#define VH_SPLIT(DSP)                                                                                                \
-    hipLaunchKernelGGL(k_pq_split<DSP>, dim3((unsigned)std::min<size_t>(8192, (n * m_sub * DSP + 255) / 256)), dim3(256), \
-                       0, s, raw, (long)n, (int)dim, (int)ds, (int)m_sub, xs, bad)
-    VH_DSP_SWITCH(dsp, VH_SPLIT)
-#undef VH_SPLIT
-    VH_HIP(hipGetLastError());
-    uint32_t nonfinite = 0;
-    VH_HIP(hipMemcpyAsync(&nonfinite, bad, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    VH_HIP(hipStreamSynchronize(s));
-    if (nonfinite) return set_error(VHIP_ERR_INVALID_CONFIG, "data contains non-finite values");
+    auto shrink = [&]() {  // false when nothing is left to shrink
+        if (group > 1) group = (group + 1) / 2;
+        else if (slab > slab_min) slab = std::max(slab_min, slab / 2);
+        else return false;
+        return true;
+    };
+    const size_t limit = pq_train_limit(layout(group).total);
+    while (layout(group).total > limit && shrink()) {}
+    int rc = mem.ensure(ordinal, layout(group).total);
+    while (rc != VHIP_OK && shrink()) rc = mem.ensure(ordinal, layout(group).total);
+    VH_CHECK(rc);
+    clear_error();
+    group = (m_sub + (m_sub + group - 1) / group - 1) / ((m_sub + group - 1) / group);  // groups of like size
+    // Only the widest kernel can need more than 64 KB of LDS.  Its limit is shared by every thread that
+    // trains, so it is set to the most that any cluster count needs, not to this call's.
     const size_t lds = pq_sums_lds(dsp, ek);
-    // Only the widest kernel can need more than 64 KB.  Its limit is shared by every thread that trains, so
-    // it is set to the most that any cluster count needs, not to this call's.
     if (dsp == 32)
         VH_HIP(hipFuncSetAttribute((const void *)k_pq_sums<32>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)pq_sums_lds(32, kPqMaxK)));
-    std::vector<uint32_t> on(m_sub, 1u);
-    std::vector<float> sh(m_sub * ek);
-    for (size_t it = 0; it < max_iters; ++it) {
+    for (size_t m0 = 0; m0 < m_sub; m0 += group) {
+        const size_t g = std::min(group, m_sub - m0);
+        const size_t per = pq_sum_points(ordinal, n, g);
+        const int parts = (int)((n + per - 1) / per);
+        const PqGroupMem L(n, dim, slab, g, ek, dsp, (size_t)parts);
+        VH_CHECK(mem.ensure(ordinal, L.total));  // a smaller last group may have more partial sums
+        char *const p0 = mem.as<char>();
+        float *raw = (float *)(p0 + L.raw), *xs = (float *)(p0 + L.xs), *cent = (float *)(p0 + L.cent),
+              *shifts = (float *)(p0 + L.shift);
+        unsigned long long *part = (unsigned long long *)(p0 + L.part);
+        uint8_t *assign = (uint8_t *)(p0 + L.assign);
+        uint32_t *count = (uint32_t *)(p0 + L.state), *devmax = count + g * ek, *active = devmax + g * ek,
+                 *bad = active + g;
+        launch_fill_u32(count, 2 * g * ek, 0u, s);
+        launch_fill_u32(active, g, 1u, s);
+        launch_fill_u32(bad, 1, 0u, s);
+        for (size_t i0 = 0; i0 < n; i0 += slab) {
+            const size_t rows = std::min(slab, n - i0);
+            VH_CHECK(st.h2d_once(raw, data + i0 * dim, rows * dim * sizeof(float), s));
+#define VH_SPLIT(DSP)                                                                                                   \
+    hipLaunchKernelGGL(k_pq_split<DSP>, dim3((unsigned)std::min<size_t>(8192, (rows * g * DSP + 255) / 256)), dim3(256), \
+                       0, s, raw, (long)rows, (long)i0, (long)n, (int)dim, (int)ds, (int)m0, (int)g, xs, bad)
+            VH_DSP_SWITCH(dsp, VH_SPLIT)
+#undef VH_SPLIT
+        }
+        VH_HIP(hipMemcpyAsync(cent, start.data() + m0 * kd, g * kd * sizeof(float), hipMemcpyHostToDevice, s));
+        VH_HIP(hipGetLastError());
+        uint32_t nonfinite = 0;
+        VH_HIP(hipMemcpyAsync(&nonfinite, bad, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        VH_HIP(hipStreamSynchronize(s));
+        if (nonfinite) return set_error(VHIP_ERR_INVALID_CONFIG, "data contains non-finite values");
+        on.assign(g, 1u);
+        sh.resize(g * ek);
+        for (size_t it = 0; it < max_iters; ++it) {
 #define VH_ITER(DSP)                                                                                                   \
     do {                                                                                                               \
-        launch_assign<L2, DSP, true>(xs, (long)n, DSP, (long)n * DSP, DSP, 1, cent, k,         \
-                                     (int)m_sub, assign, 1, (long)n, count, devmax, active, s);          \
-        hipLaunchKernelGGL(k_pq_sums<DSP>, dim3((unsigned)parts, (unsigned)m_sub), dim3(kPqThreads), lds, s,           \
-                           xs, (long)n, (long)per, cent, k, assign, count,       \
-                           devmax, part, active);                                             \
-        hipLaunchKernelGGL(k_pq_finalize<DSP>, dim3((unsigned)ceil_div((long)ek, kPqThreads / DSP), (unsigned)m_sub),  \
-                           dim3(kPqThreads), 0, s, cent, k, parts, part, count,   \
-                           devmax, shifts, active);                                                        \
+        launch_assign<L2, DSP, true>(xs, (long)n, DSP, (long)n * DSP, DSP, 1, cent, k, (int)g, assign, 1, (long)n,      \
+                                     count, devmax, active, s);                                                        \
+        hipLaunchKernelGGL(k_pq_sums<DSP>, dim3((unsigned)parts, (unsigned)g), dim3(kPqThreads), lds, s, xs, (long)n,   \
+                           (long)per, cent, k, assign, count, devmax, part, active);                                   \
+        hipLaunchKernelGGL(k_pq_finalize<DSP>, dim3((unsigned)ceil_div((long)ek, kPqThreads / DSP), (unsigned)g),      \
+                           dim3(kPqThreads), 0, s, cent, k, parts, part, count, devmax, shifts, active);               \
     } while (0)
-        VH_DSP_SWITCH(dsp, VH_ITER)
+            VH_DSP_SWITCH(dsp, VH_ITER)
 #undef VH_ITER
-        VH_HIP(hipGetLastError());
-        if (tol >= 0.0f) {  // a sub-space stops when no centroid of it moved by more than tol
-            VH_HIP(hipMemcpyAsync(sh.data(), shifts, sh.size() * sizeof(float), hipMemcpyDeviceToHost, s));
-            VH_HIP(hipStreamSynchronize(s));
-            bool changed = false, any = false;
-            for (size_t m = 0; m < m_sub; ++m) {
-                if (!on[m]) continue;
-                const float mx = *std::max_element(sh.begin() + m * ek, sh.begin() + (m + 1) * ek);
-                if (mx <= tol) {
-                    on[m] = 0;
-                    changed = true;
-                } else {
-                    any = true;
+            VH_HIP(hipGetLastError());
+            if (tol >= 0.0f) {  // a sub-space stops when no centroid of it moved by more than tol
+                VH_HIP(hipMemcpyAsync(sh.data(), shifts, sh.size() * sizeof(float), hipMemcpyDeviceToHost, s));
+                VH_HIP(hipStreamSynchronize(s));
+                bool changed = false, any = false;
+                for (size_t m = 0; m < g; ++m) {
+                    if (!on[m]) continue;
+                    const float mx = *std::max_element(sh.begin() + m * ek, sh.begin() + (m + 1) * ek);
+                    if (mx <= tol) {
+                        on[m] = 0;
+                        changed = true;
+                    } else {
+                        any = true;
+                    }
+                }
+                if (!any) break;
+                if (changed) {
+                    VH_HIP(hipMemcpyAsync(active, on.data(), g * sizeof(uint32_t), hipMemcpyHostToDevice, s));
+                    VH_HIP(hipStreamSynchronize(s));
                 }
             }
-            if (!any) break;
-            if (changed) {
-                VH_HIP(hipMemcpyAsync(active, on.data(), m_sub * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-                VH_HIP(hipStreamSynchronize(s));
-            }
         }
+        fin.resize(g * kd);
+        VH_HIP(hipMemcpyAsync(fin.data(), cent, fin.size() * sizeof(float), hipMemcpyDeviceToHost, s));
+        VH_HIP(hipStreamSynchronize(s));
+        for (size_t m = 0; m < g; ++m)
+            for (size_t j = 0; j < ek; ++j)
+                std::copy(fin.begin() + (m * ek + j) * dsp, fin.begin() + (m * ek + j) * dsp + ds,
+                          out_codebooks + ((m0 + m) * ks + j) * ds);
     }
-    std::vector<float> fin(m_sub * kd);
-    VH_HIP(hipMemcpyAsync(fin.data(), cent, fin.size() * sizeof(float), hipMemcpyDeviceToHost, s));
-    VH_HIP(hipStreamSynchronize(s));
-    for (size_t m = 0; m < m_sub; ++m)
-        for (size_t j = 0; j < ek; ++j)
-            std::copy(fin.begin() + (m * ek + j) * dsp, fin.begin() + (m * ek + j) * dsp + ds,
-                      out_codebooks + (m * ks + j) * ds);
     return VHIP_OK;
 }
 
