@@ -58,6 +58,19 @@ def test_sub_spaces_stop_by_themselves(vh):
     np.testing.assert_allclose(got[1], c, rtol=1e-6)
 
 
+def test_a_nan_centroid_does_not_keep_a_sub_space_running(vh):
+    """A NaN centroid's shift is NaN; as in the general engine it takes no part in the largest shift, so the
+    sub-space stops after the first iteration, when the others moved by less than the tolerance."""
+    rng = np.random.default_rng(6)
+    x = rng.integers(0, 100, (2000, 2)).astype(np.float32)
+    x[0, 0] = np.nan  # nearest to no centroid: goes to the first
+    init = np.concatenate([[[np.nan, 0.0]], x[1:8]]).astype(np.float32)[None]
+    got = vh.ProductQuantizer.train(x, 2, 1, 8, 30, 1e4, init_codebooks=init).codebooks.reshape(8, 2)
+    c, _, r = vh.KMeansState(x).fit(8, 30, 1e4, init=init[0])
+    assert r[2] == 1
+    np.testing.assert_allclose(got[1:], c[1:], rtol=1e-6)
+
+
 def test_threads_train_with_different_cluster_counts(vh):
     """Trainings that need 39, 65 and 98 KB of LDS a workgroup, at the same time."""
     from concurrent.futures import ThreadPoolExecutor

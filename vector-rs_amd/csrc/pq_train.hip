@@ -501,7 +501,8 @@ int pq_train_batched(int ordinal, const float *data, size_t n, size_t dim, size_
                 bool changed = false, any = false;
                 for (size_t m = 0; m < g; ++m) {
                     if (!on[m]) continue;
-                    const float mx = *std::max_element(sh.begin() + m * ek, sh.begin() + (m + 1) * ek);
+                    float mx = 0.0f;  // a NaN shift takes no part
+                    for (size_t j = 0; j < ek; ++j) mx = std::max(mx, sh[m * ek + j]);
                     if (mx <= tol) {
                         on[m] = 0;
                         changed = true;
