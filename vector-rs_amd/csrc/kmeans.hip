@@ -1184,21 +1184,18 @@ int vhip_kmeans_read(vhip_kmeans *K, float *centroids, int32_t *assign, int64_t 
     std::lock_guard<std::mutex> lock(K->mu);
     VH_CHECK(open_device(K->dev));
     hipStream_t s = K->stream;
-    // the inertia's sum first, so that one wait covers it and the copies
+    const size_t cbytes = K->k * K->dim * sizeof(float);
+    const bool unpad = centroids && K->k && K->dim != K->dpad;
+    if (unpad) VH_CHECK(K->rows_out.ensure(K->dev, cbytes));  // before any copy to this call's own buffers
     constexpr int kInertiaParts = 256;
-    std::vector<double> part;
     if (inertia && K->assigned) {
-        part.resize(kInertiaParts);
         const size_t chunk = (K->n + kInertiaParts - 1) / kInertiaParts;
         hipLaunchKernelGGL(k_sum_partial, dim3(kInertiaParts), dim3(256), 0, s, K->inertia.as<float>(), K->n, chunk,
                            K->partial.as<double>());
         VH_HIP(hipGetLastError());
-        VH_HIP(hipMemcpyAsync(part.data(), K->partial.p, kInertiaParts * sizeof(double), hipMemcpyDeviceToHost, s));
     }
-    const size_t cbytes = K->k * K->dim * sizeof(float);
     const void *crows = K->craw.p;
-    if (centroids && K->k && K->dim != K->dpad) {
-        VH_CHECK(K->rows_out.ensure(K->dev, cbytes));
+    if (unpad) {
         const size_t blocks = std::min<size_t>(4096, (K->k * K->dim + 255) / 256);
         hipLaunchKernelGGL(k_rows_unpad, dim3((unsigned)blocks), dim3(256), 0, s, K->craw.as<float>(), K->k * K->dim,
                            (int)K->dim, (int)K->dpad, K->rows_out.as<float>());
@@ -1212,8 +1209,13 @@ int vhip_kmeans_read(vhip_kmeans *K, float *centroids, int32_t *assign, int64_t 
         VH_CHECK(K->stager.d2h(centroids, crows, cbytes, s));
     else if (want_assign)
         VH_CHECK(K->stager.d2h(assign, K->assign.p, K->n * sizeof(int32_t), s));
+    std::vector<double> part;
     std::vector<int32_t> c32;
     std::vector<float> sh;
+    if (inertia && K->assigned) {
+        part.resize(kInertiaParts);
+        VH_HIP(hipMemcpyAsync(part.data(), K->partial.p, kInertiaParts * sizeof(double), hipMemcpyDeviceToHost, s));
+    }
     if (K->assigned && K->k && counts) {
         c32.resize(K->k);
         VH_HIP(hipMemcpyAsync(c32.data(), K->counts.p, K->k * sizeof(int32_t), hipMemcpyDeviceToHost, s));
