@@ -198,3 +198,24 @@ def test_too_large_for_the_array_is_an_error(vh):
     dq2 = vh.DeviceBuffer.from_host(base[:2, :64].copy())
     small.search_batch_device_noalloc(dq2.ptr, 2, 4, di.ptr, dd.ptr)
     assert di.to_host(np.empty((2, 4), np.uint32))[:, 0].tolist() == [0, 1]
+
+
+def test_longest_rows_that_fit_the_array(vh, oracle):
+    """Rows of 43,520 floats at k = 944: one query's buffers and its re-run's fill the array to the last
+    kilobyte.  They hold no norms or error bounds for a metric that has none."""
+    rng = np.random.default_rng(4)
+    base = rng.uniform(-1, 1, (1000, 43_520)).astype(np.float32)
+    q = rng.uniform(-1, 1, (2, 43_520)).astype(np.float32)
+    eng = vh.CudaKnnEngine(base, 43_520, vh.DistanceMetric.Manhattan)
+    dq = vh.DeviceBuffer.from_host(q)
+    out = []
+    for search in (eng.search_batch_device_noalloc, eng.search_batch_device):
+        di, dd = vh.DeviceBuffer(2 * 944 * 4), vh.DeviceBuffer(2 * 944 * 4)
+        search(dq.ptr, 2, 944, di.ptr, dd.ptr)
+        vh.synchronize()
+        out.append((di.to_host(np.empty((2, 944), np.uint32)), dd.to_host(np.empty((2, 944), np.float32))))
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    np.testing.assert_array_equal(out[0][1], out[1][1])
+    for r in range(2):
+        ref = oracle.distance_rows("l1", np.repeat(q[r:r + 1], 944, 0), base[out[0][0][r]])
+        np.testing.assert_allclose(out[0][1][r], ref, rtol=1e-4)

@@ -330,7 +330,7 @@ static bool want_fp4_copy(size_t bytes) {
 }
 
 // One batch of prepared queries: the rows the scan kernels read (shifted for squared L2), their
-// norms and selection error bounds (null for the non-GEMM metrics), and the unshifted rows of
+// norms and selection error bounds (both null for the non-GEMM metrics), and the unshifted rows of
 // the direct-form passes (qpad itself when the engine keeps no shift).
 struct QueryRows {
     const float *qpad, *qnorm, *qerr, *qraw;
@@ -527,8 +527,10 @@ static RerunMem carve_rerun(Arena &A, const vhip_knn *E, size_t nidx, size_t per
     r.fr = A.take<float>(m_pad * E->dpad);
     if (!direct) {
         r.fq = A.take<float>(m_pad * E->dpad);
-        r.fn = A.take<float>(m_pad);
-        r.fe = A.take<float>(m_pad);
+        if (is_gemm_metric(E->metric)) {
+            r.fn = A.take<float>(m_pad);
+            r.fe = A.take<float>(m_pad);
+        }
     }
     r.F = carve_run(A, E, per_batch, kc_run, cap, with_cand);
     return r;
@@ -577,14 +579,16 @@ static int rerun_queries(vhip_knn *E, const QueryRows &Q, const std::vector<uint
         F.qraw = R.fr;
         if (!direct) {
             launch_fill(R.fq + (size_t)m * dp, (m_pad - m) * E->dpad, 0.0f, s);
-            launch_fill(R.fn + m, m_pad - m, 0.0f, s);
-            launch_fill(R.fe + m, m_pad - m, 0.0f, s);
             launch_gather_rows(Q.qpad, di, (size_t)m, dp, R.fq, s);
-            launch_gather_rows(Q.qnorm, di, (size_t)m, 1, R.fn, s);
-            if (Q.qerr) launch_gather_rows(Q.qerr, di, (size_t)m, 1, R.fe, s);
             F.qpad = R.fq;
-            F.qnorm = R.fn;
-            F.qerr = Q.qerr ? R.fe : nullptr;
+            if (is_gemm_metric(E->metric)) {
+                launch_fill(R.fn + m, m_pad - m, 0.0f, s);
+                launch_fill(R.fe + m, m_pad - m, 0.0f, s);
+                launch_gather_rows(Q.qnorm, di, (size_t)m, 1, R.fn, s);
+                launch_gather_rows(Q.qerr, di, (size_t)m, 1, R.fe, s);
+                F.qnorm = R.fn;
+                F.qerr = R.fe;
+            }
         }
         VH_CHECK(run_rounds(E, F, m, k, kc_run, cap, direct, small_plan(E, per_batch, direct), R.F, max_rows,
                             fixed == nullptr));
@@ -821,7 +825,7 @@ static BatchMem carve_batch(Arena &A, const vhip_knn *E, size_t m, int kc, int c
     const size_t m_pad = round_up(m, kTileCols);
     BatchMem b{};
     b.qpad = A.take<float>(m_pad * E->dpad);
-    b.qnorm = A.take<float>(m_pad);
+    b.qnorm = is_gemm_metric(E->metric) ? A.take<float>(m_pad) : nullptr;
     b.qerr = is_gemm_metric(E->metric) ? A.take<float>(m_pad) : nullptr;
     b.qraw = E->shifted ? A.take<float>(m_pad * E->dpad) : nullptr;
     b.B = carve_run(A, E, m, kc, cap, true);
