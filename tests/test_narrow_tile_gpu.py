@@ -1,5 +1,5 @@
-"""The narrow resident-tile MFMA search kernel at every kind of row width it takes (129 to 896 floats):
-odd and even chunk counts, widths with padding, row ranges that end inside a 512-row stage and query
+"""The narrow resident-tile MFMA search kernel at row widths it takes (129 to 896 floats): every odd count of
+32-float chunks, even ones, widths with padding, row ranges that end inside a 512-row stage and query
 tiles that end inside 32 columns."""
 import numpy as np
 import pytest
@@ -12,7 +12,8 @@ NAMES = {"l2": "L2Squared", "dot": "DotProduct", "cosine": "CosineSimilarity"}
 
 
 @pytest.mark.parametrize("metric", ["l2", "dot", "cosine"])
-@pytest.mark.parametrize("dim", [129, 160, 191, 200, 288, 300, 352, 416, 420, 500, 545, 608, 672, 700, 736, 800, 831, 865])
+@pytest.mark.parametrize("dim", [129, 160, 191, 200, 288, 300, 352, 416, 420, 480, 500, 544, 545, 608, 672, 700,
+                                 736, 800, 831, 864, 865, 896])
 def test_row_widths(oracle, metric, dim):
     import vector_hip as vh
 

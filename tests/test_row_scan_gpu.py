@@ -1,14 +1,22 @@
-"""Small query batches under the vector-ALU metrics and packed Hamming (knn_rows.hip).
+"""The row-per-lane scans (knn_rows.hip): the vector-ALU metrics at every batch size, packed Hamming in
+small batches, and the fp4 Hamming round plans.
 
-A score's terms are summed in the batch kernels' order, so a query gets the same ids and the same
-distances, bit for bit, whether it is searched in a small batch or within a large one; the large
-batches are held to the oracle elsewhere.  Sizes sit at the edges of the kernels: query tiles of 4 and
-16, the 64-query limit, 32-dimension chunks and the two chunk widths of the batch kernel, workgroups
-of 256 rows, the 8,192-row first round and one more round."""
+A score's terms are summed in one order whatever the batch, so a query gets the same ids and the same
+distances, bit for bit, whether it is searched alone or within a large batch.  Batches of up to 128
+queries take the small-batch round plan and count candidates on spread counters; the batch of 300 they
+are compared with takes the growing plan, and is held to the oracle.  Sizes sit at the edges of the
+kernels: query tiles of 4 and 16, 128 and 129 queries, 32-dimension chunks and halves of 16, the two
+sums' boundary at 64 and 128 dimensions, workgroups of 256 rows, bases of one dense round (16,384 rows
+in the small plan, 2,048 in the other) and of several."""
 import numpy as np
 import pytest
 
+from knn_check import check_knn
+
 pytestmark = pytest.mark.gpu
+
+ORACLE = {"Manhattan": "l1", "Minkowski": "minkowski", "Chebyshev": "linf", "Hamming": "hamming",
+          "Mahalanobis": "mahalanobis", "Jaccard": "jaccard", "Hellinger": "hellinger"}
 
 
 @pytest.fixture(scope="module")
@@ -19,45 +27,54 @@ def vh():
     return vector_hip
 
 
-@pytest.mark.parametrize("metric", ["Manhattan", "Minkowski", "Chebyshev", "Hamming", "Mahalanobis", "Jaccard",
-                                    "Hellinger"])
+@pytest.mark.parametrize("metric", list(ORACLE))
 @pytest.mark.parametrize("n,dim,k", [(3, 5, 10), (257, 32, 1), (8193, 33, 7), (20_001, 65, 100), (16_385, 128, 10),
                                      (140_000, 129, 10), (9000, 200, 300)])
-def test_small_batches_equal_large_ones(vh, metric, n, dim, k):
+def test_every_batch_size_agrees(vh, oracle, metric, n, dim, k):
     rng = np.random.default_rng(n + dim)
     base = rng.uniform(-1, 1, (n, dim)).astype(np.float32)
     base[rng.integers(0, n, n // 3)] = base[rng.integers(0, n, n // 3)]  # equal rows: ties by id
     if metric == "Hamming":
         base = np.round(base * 2)
-    q = np.concatenate([base[:2], rng.uniform(-1, 1, (78, dim)).astype(np.float32)])
+    q = np.concatenate([base[:2], rng.uniform(-1, 1, (298, dim)).astype(np.float32)])
     eng = vh.CudaKnnEngine(base, dim, vh.DistanceMetric[metric])
     ids, dist, lens = eng.search_batch_arrays(q, k)
     kk = min(k, n)
-    for nq in (1, 4, 5, 16, 17, 64):
+    held = [0, 1, 2, 7, 128, 299]
+    # sums of up to 200 terms in another order than the oracle's, and cbrt / sqrt of them
+    check_knn(oracle, base, q[held], ids[held], dist[held], k, ORACLE[metric], rtol=2e-5, atol=2e-6)
+    for nq in (1, 4, 5, 16, 17, 64, 128, 129):
         i2, d2, l2 = eng.search_batch_arrays(q[:nq], k)
         np.testing.assert_array_equal(i2[:, :kk], ids[:nq, :kk])
         np.testing.assert_array_equal(d2[:, :kk], dist[:nq, :kk])
         np.testing.assert_array_equal(l2, lens[:nq])
 
 
+# one dense round in the small plan and several in the other; dense and filter rounds in both
+@pytest.mark.parametrize("n,share", [(9000, 0.999), (60_000, 0.9998), (60_000, 0.5)])
 @pytest.mark.parametrize("metric", ["Manhattan", "Minkowski"])
-def test_rows_and_queries_with_nan(vh, metric):
-    """A row with a NaN never appears, a query with one finds nothing, in small and large batches alike."""
+def test_rows_and_queries_with_nan(vh, metric, n, share):
+    """A row with a NaN never appears and a query with one finds nothing, in small and large batches alike,
+    whether the rows without are fewer than k or many, in the first round or in later ones."""
     rng = np.random.default_rng(3)
-    base = rng.uniform(-1, 1, (9000, 40)).astype(np.float32)
-    bad = rng.random(9000) < 0.999
-    base[bad, 7] = np.nan  # fewer finite rows than k
-    q = rng.uniform(-1, 1, (80, 40)).astype(np.float32)
+    base = rng.uniform(-1, 1, (n, 40)).astype(np.float32)
+    bad = rng.random(n) < share
+    base[bad, 7] = np.nan
+    q = rng.uniform(-1, 1, (300, 40)).astype(np.float32)
     q[1, 0] = np.nan
     eng = vh.CudaKnnEngine(base, 40, vh.DistanceMetric[metric])
     ids, dist, _ = eng.search_batch_arrays(q, 30)
     good = np.flatnonzero(~bad)
-    assert 0 < good.size < 30
-    for r in (0, 2, 79):
-        assert sorted(ids[r, :good.size]) == good.tolist()
-        assert np.all(ids[r, good.size:] == 0xFFFFFFFF) and np.all(np.isnan(dist[r, good.size:]))
+    assert good.size > 0
+    found = min(30, good.size)
+    p = 1 if metric == "Manhattan" else 3
+    for r in (0, 2, 299):
+        assert np.all(np.isin(ids[r, :found], good)) and len(set(ids[r, :found].tolist())) == found
+        assert np.all(ids[r, found:] == 0xFFFFFFFF) and np.all(np.isnan(dist[r, found:]))
+        want = np.sort((np.abs(base[good].astype(np.float64) - q[r]) ** p).sum(1) ** (1 / p))[:found]
+        np.testing.assert_allclose(dist[r, :found], want, rtol=1e-5)  # 40 terms in 32 bits
     assert np.all(ids[1] == 0xFFFFFFFF)
-    for nq in (2, 16, 33):
+    for nq in (2, 16, 33, 128, 129):
         i2, d2, _ = eng.search_batch_arrays(q[:nq], 30)
         np.testing.assert_array_equal(i2, ids[:nq])
         np.testing.assert_array_equal(d2, dist[:nq])
