@@ -9,13 +9,14 @@
 //      centroids are wave-uniform and come through the scalar cache, so an element costs one subtract
 //      and one multiply-add.  The scores are the direct form the general engine's fix-up computes
 //      (sequential over the dimensions, lowest index among equal ones), so every assignment is the one
-//      its certified MFMA scan ends with;
+//      its certified MFMA scan ends with.  (Its small-set kernel, for up to 1e6 (point, centroid) pairs,
+//      adds slices of a row, so there a point between two centroids may go by another last bit);
 //   2. k_pq_sums -- deviations x - c in 64-bit fixed point with the cluster's own scale, as in
 //      kmeans.hip, summed with LDS integer atomics (exact in any order) and written per workgroup;
 //   3. k_pq_finalize -- the workgroups' sums added up, new = old + sum / count, the centroid's shift.
 // Bound: the vector ALUs in the assignment.  65,536 x 128 points, 8 sub-spaces of 256 centroids, 10
 // iterations, host data in, codebooks out: 21 ms by sub-space k-means, 3.3 here (1.7 of it the upload and
-// allocations); an assignment of all sub-spaces takes 129 us (94 at the rate of its subtracts and
+// allocations, which vary by box); an assignment of all sub-spaces takes 129 us (94 at the rate of its subtracts and
 // multiply-adds), the sums 18, the new centroids 8.  Encoding the same points: 524 us -> 134.
 #include <algorithm>
 #include <cmath>

@@ -64,8 +64,16 @@ inline bool small_batch(int nq, int dpad, size_t n) {
            (nq <= kSmallCols || (nq <= 4 * kSmallCols && (n <= kSmallBaseRows || dpad <= 128)));
 }
 // Batches of at most kValuSmallQueries queries under the metrics that run on the vector ALUs take the
-// small-batch round plan; batches of at most kHamSmallQueries over packed codes are scanned with
-// popcounts (knn_rows.hip: the figures of both sides).
+// small-batch round plan: 128 is the number of spread counters (kSmallPadQueries), and the plan is still
+// ahead there.  Whole searches, k = 10, growing plan -> small plan, microseconds:
+//   L1 128 dimensions      4 queries    32           64           128
+//     9,000 rows           63 -> 38     69 -> 40     72 -> 42     73 -> 48
+//     150,000              99 -> 65     131 -> 93    165 -> 109   211 -> 156
+//     500,000              125 -> 88    199 -> 143   275 -> 212   413 -> 361
+//   Jaccard 500 dimensions
+//     60,000               206 -> 122   250 -> 194   349 -> 351   618 -> 496
+// Batches of at most kHamSmallQueries over packed codes are scanned with popcounts (knn_rows.hip: the
+// figures of both sides).
 constexpr int kValuSmallQueries = 128;
 constexpr int kHamSmallQueries = 16;
 // Packed Hamming on the fp4 matrix cores takes the small-batch round plan (three rounds at 4M rows where
