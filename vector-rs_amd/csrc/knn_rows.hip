@@ -71,7 +71,8 @@ __device__ __forceinline__ bool scan_tile(const RowScanArgs &a, int &group, int 
     const unsigned b = blockIdx.x;
     if (a.spread) {
         const unsigned seq = b >> 3, per_xcd = (unsigned)(a.n_groups + 7) / 8u;  // row groups of an XCD
-        const unsigned first = seq / (per_xcd * (unsigned)a.chunk) * (unsigned)a.chunk;
+        const unsigned first =
+            a.chunk < a.n_qtiles ? seq / (per_xcd * (unsigned)a.chunk) * (unsigned)a.chunk : 0u;
         const unsigned tiles = min((unsigned)a.chunk, (unsigned)a.n_qtiles - first);
         const unsigned at = seq - per_xcd * first;
         group = (int)(at / tiles * 8u + (b & 7u));
